@@ -29,7 +29,8 @@ HBM_PEAK_GBS = 8000.0
 RBGS_BYTES_PER_VOXEL_SWEEP = 12.0  # read p, read rhs, write p
 RBGS_KERNELS = {1: ("k_rbgs_pass", "RBGS colour pass, two per sweep", "rbgs_pass_traffic.json"),
                 2: ("k_rbgs_fused", "RBGS fused sweep, one per sweep", "rbgs_fused_traffic.json"),
-                3: ("k_rbgs_pair", "RBGS row-pair fused sweep, one per sweep", "rbgs_pair_traffic.json")}
+                3: ("k_rbgs_pair", "RBGS row-pair fused sweep, one per sweep", "rbgs_pair_traffic.json"),
+                4: ("k_rbgs_tile", "RBGS tile sweeps, two to five per launch", "")}
 # compulsory bytes per voxel of the non-solve part of a substep of this
 # workload: cooling 8, vorticity 24, buoyancy 12, divergence 16, update 28,
 # advection 40 (T, U, V, W, density)
@@ -543,12 +544,15 @@ def report(a, s, gen, parts, L, LT, warm):
     value = N3 * tot_sub / elapsed
     ms_per_step = elapsed * 1e3 / a.steps
     # algorithmic bytes of the timed sweeps over their device time; per
-    # launch that is 12 B/voxel (fused sweep) or 6 B/voxel (colour pass)
+    # launch that is 12 B/voxel (fused sweep, or tile sweeps, which read and
+    # write the planes once for all sweeps of a launch) or 6 B/voxel (colour
+    # pass)
     avg_launch_s = (tot_rbgs_ms / 1e3) / max(1, tot_launch)
-    achieved = (RBGS_BYTES_PER_VOXEL_SWEEP * N3 * tot_timed_sweeps / (tot_rbgs_ms / 1e3) / 1e9
+    passes = tot_launch if kernel_kind == 4 else tot_timed_sweeps
+    achieved = (RBGS_BYTES_PER_VOXEL_SWEEP * N3 * passes / (tot_rbgs_ms / 1e3) / 1e9
                 if tot_rbgs_ms > 0 else 0.0)
     kname, kdesc, kfile = RBGS_KERNELS.get(kernel_kind, ("?", "?", ""))
-    algo_bytes = N3 * (FIXED_BYTES_PER_VOXEL * tot_sub + 12.0 * tot_iters
+    algo_bytes = N3 * (FIXED_BYTES_PER_VOXEL * tot_sub + 12.0 * (passes if kernel_kind == 4 else tot_iters)
                        + RESIDUAL_BYTES_PER_VOXEL * tot_checks)
     step_gbs = algo_bytes / elapsed / 1e9
 
@@ -607,6 +611,7 @@ def report(a, s, gen, parts, L, LT, warm):
             "traffic": traffic,
             "avg_launch_us": avg_launch_s * 1e6,
             "launches": tot_launch,
+            "us_per_sweep": tot_rbgs_ms * 1e3 / max(1, tot_timed_sweeps),
             "timing_pass_ms_per_step": LT["elapsed"] * 1e3 / a.steps,
         },
         "cpu_baseline": cpu,

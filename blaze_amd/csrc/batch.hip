@@ -4,9 +4,9 @@
 // and the warm start's network of all scenes run as single launches over
 // tables of grids (k_rbgs_fused_multi, k_residual_multi, k_pupdate_multi,
 // k_advect_multi, NetMulti), so small grids share the GPU instead of being
-// launch-bound one by one. The sweep kernel's tile parameters (slab groups
-// in flight, waves per block) come from an autotuner that times each
-// candidate on the batch itself.
+// launch-bound one by one. The sweeps are those of k_sweep.hip (several per
+// launch) or a one-sweep variant that the autotuner found faster on the
+// batch itself.
 //
 // No reference counterpart (the reference runs one scene per process,
 // src/main.cu:72-117). Each scene computes exactly what blz_step computes
@@ -109,6 +109,7 @@ struct Batch {
     int fs_blocks = 0, rs_blocks = 0;
     int every = 10;
     int variant = 103;
+    int family = 0; // tiles of variant VARIANT_TILES, one family for all scenes
     int nodes = 0;
     double capture_ms = 0.0, step_ms = 0.0;
     double tune_ms[NTUNE] = {};
@@ -116,6 +117,8 @@ struct Batch {
 
     ~Batch();
     int init(const blz_settings* st, int n);
+    int blocks_of(const Solver& s, int v) const;
+    int sweep_batch(hipStream_t st, const FusedScene* a, const FusedScene* b, int n, int blocks, int sweeps);
     int build_tables(int v);
     int build_judge_tables();
     int capture(int which);
@@ -131,7 +134,10 @@ struct Batch {
 // fused (one row per wave) and row-pair candidates; waves per block = the
 // hundreds digit
 static const int kVariants[NTUNE] = {102, 103, 202, 203, 402, 403, 1103, 1104, 1203, 1204};
-static int wpb_of(int v) { return (v / 100) % 10; }
+static int wpb_of(int v) { return v == VARIANT_TILES ? 1 : (v / 100) % 10; }
+// several sweeps per launch need at least two launches of two sweeps between
+// two checks
+static bool tiles_fit(int every) { return every >= 4; }
 // sweeps per graph of a step's later sweeps (about 30 ms of sweeps of the
 // 64-scene benchmark batch)
 constexpr int CHUNK_SWEEPS = 160;
@@ -209,7 +215,37 @@ int Batch::init(const blz_settings* st, int n) {
         BLZ_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         join.push_back(e);
     }
-    return build_tables(variant);
+    // the tiles as for one grid (tile_family), by the tiles of all scenes
+    for (family = 0; family < TILE_FAMILIES - 1; ++family) {
+        long long tiles = 0;
+        for (blz_solver* h : sc) tiles += tile_count(family, h->s.W, h->s.H);
+        if (tiles <= 256) break;
+    }
+    return build_tables(tiles_fit(every) ? VARIANT_TILES : variant);
+}
+
+// sweep blocks of one scene: tiles, or waves of the one-sweep variants
+int Batch::blocks_of(const Solver& s, int v) const {
+    if (v == VARIANT_TILES) return tile_count(family, s.W, s.H);
+    return v >= 1000 ? pair_waves(s) : fused_waves(s);
+}
+
+// an even number of sweeps of every scene of two tables (a: there, b: back)
+int Batch::sweep_batch(hipStream_t st, const FusedScene* a, const FusedScene* b, int n, int blocks, int sweeps) {
+    if (variant == VARIANT_TILES) {
+        int launches = 0, left = 0;
+        if (int e = launch_tile_sweeps(st, family, a, b, n, blocks, sweeps, &launches, &left)) return e;
+        if (left) {
+            set_error("batch: sweeps left over by the tile launches");
+            return BLZ_E_INVALID;
+        }
+        return BLZ_OK;
+    }
+    for (int l = 0; l < sweeps / 2; ++l) {
+        if (int e = launch_fused_multi(st, variant, a, n, blocks)) return e;
+        if (int e = launch_fused_multi(st, variant, b, n, blocks)) return e;
+    }
+    return BLZ_OK;
 }
 
 int Batch::build_tables(int v) {
@@ -220,27 +256,11 @@ int Batch::build_tables(int v) {
     int fb = 0, rb = 0;
     for (int q = 0; q < n; ++q) {
         Solver& s = sc[q]->s;
-        const unsigned pb = (unsigned)(s.Np * 4);
         const float dt = s.s.dt;
-        const int nw = v >= 1000 ? pair_waves(s) : fused_waves(s);
+        const int nw = blocks_of(s, v);
         for (int h = 0; h < 2; ++h) {
             FusedScene& e = fs_h[h * n + q];
-            const unsigned src = h == 0 ? 0u : 4u * pb, dst = h == 0 ? 4u * pb : 0u;
-            e.base = s.prb;
-            e.nbytes = (unsigned)(s.prb_floats * 4);
-            e.srcR = src;
-            e.srcB = src + pb;
-            e.rhsR = 2u * pb;
-            e.rhsB = 3u * pb;
-            e.dstR = dst;
-            e.dstB = dst + pb;
-            e.W = s.W;
-            e.H = s.H;
-            e.D = s.D;
-            e.Wp = s.L.Wp;
-            e.Hp = s.L.Hp;
-            e.scale = (s.s.density * s.dx * s.dx) / dt; // gs_solve_kernel :530
-            e.stop = &s.ctl[0].done;
+            e = h == 0 ? sweep_scene(s, dt, 0, 4, &s.ctl[0].done) : sweep_scene(s, dt, 4, 0, &s.ctl[0].done);
             e.first_block = fb;
             e.nwaves = nw;
         }
@@ -528,14 +548,8 @@ int Batch::enqueue_step(hipStream_t st) {
         // corrected pressure (home planes), the same on the uncorrected one
         // (judge planes), both residuals, the decisions and restores
         const int nw = (int)warm_q.size();
-        for (int l = 0; l < every / 2; ++l) {
-            if (int e = launch_fused_multi(st, variant, fsw, nw, w_fs_blocks)) return e;
-            if (int e = launch_fused_multi(st, variant, fsw + nw, nw, w_fs_blocks)) return e;
-        }
-        for (int l = 0; l < every / 2; ++l) {
-            if (int e = launch_fused_multi(st, variant, fsj, nw, w_fs_blocks)) return e;
-            if (int e = launch_fused_multi(st, variant, fsj + nw, nw, w_fs_blocks)) return e;
-        }
+        if (int e = sweep_batch(st, fsw, fsw + nw, nw, w_fs_blocks, every)) return e;
+        if (int e = sweep_batch(st, fsj, fsj + nw, nw, w_fs_blocks, every)) return e;
         if (int e = launch_residual_partials_multi(st, rsw, nw, w_rs_blocks)) return e;
         if (int e = launch_residual_partials_multi(st, rsj, nw, w_rs_blocks)) return e;
         if (int e = launch_ws_judge_multi(st, js, nw, w_restore_blocks, every)) return e;
@@ -564,10 +578,7 @@ int Batch::enqueue_step(hipStream_t st) {
             ++cuts;
         }
         ++batches;
-        for (int l = 0; l < every / 2; ++l) {
-            if (int e = launch_fused_multi(st, variant, fs, n, fs_blocks)) return e;
-            if (int e = launch_fused_multi(st, variant, fs + n, n, fs_blocks)) return e;
-        }
+        if (int e = sweep_batch(st, fs, fs + n, n, fs_blocks, every)) return e;
         if (int e = launch_residual_multi(st, rs, n, rs_blocks, every, 0)) return e;
         // warm_start = N >= 2: each scene's learned correction every N sweeps
         std::vector<char> again(n, 0);
@@ -604,16 +615,10 @@ int Batch::enqueue_step(hipStream_t st) {
             }
             if (joint_fwd)
                 if (int e = joint_forward_and_finish(st)) return e;
-            for (int l = 0; l < every / 2; ++l) {
-                if (int e = launch_fused_multi(st, variant, fsw, nw, w_fs_blocks)) return e;
-                if (int e = launch_fused_multi(st, variant, fsw + nw, nw, w_fs_blocks)) return e;
-            }
+            if (int e = sweep_batch(st, fsw, fsw + nw, nw, w_fs_blocks, every)) return e;
             if (int e = launch_residual_partials_multi(st, rsw, nw, w_rs_blocks)) return e;
             if (int e = launch_ws_judge_pred_multi(st, js, nw, every)) return e;
-            for (int l = 0; l < every / 2; ++l) {
-                if (int e = launch_fused_multi(st, variant, fsj2, nw, w_fs_blocks)) return e;
-                if (int e = launch_fused_multi(st, variant, fsj2 + nw, nw, w_fs_blocks)) return e;
-            }
+            if (int e = sweep_batch(st, fsj2, fsj2 + nw, nw, w_fs_blocks, every)) return e;
             if (int e = launch_residual_partials_multi(st, rsj2, nw, w_rs_blocks)) return e;
             if (int e = launch_ws_judge_fin_multi(st, js, nw, w_restore_blocks, every)) return e;
             for (int q : warm_q) it[q] += every;
@@ -845,22 +850,21 @@ int Batch::autotune(int sweeps, int* best) {
     int bestv = variant;
     double bestms = 1e30;
     int rc = BLZ_OK;
-    for (int c = 0; c < NTUNE && !rc; ++c) {
-        const int v = kVariants[c];
+    // the one-sweep candidates (reported), then several sweeps per launch
+    for (int c = 0; c < NTUNE + (tiles_fit(every) ? 1 : 0) && !rc; ++c) {
+        const int v = c < NTUNE ? kVariants[c] : VARIANT_TILES;
+        const int count = std::max(sweeps, v == VARIANT_TILES ? every & ~1 : 2);
         if ((rc = build_tables(v))) break;
-        // one untimed pair, then the timed sweeps
-        if ((rc = launch_fused_multi(root, v, fs, n, fs_blocks)) || (rc = launch_fused_multi(root, v, fs + n, n, fs_blocks)))
-            break;
+        // one untimed round, then the timed sweeps
+        if ((rc = sweep_batch(root, fs, fs + n, n, fs_blocks, v == VARIANT_TILES ? count : 2))) break;
         (void)hipEventRecord(e0, root);
-        for (int l = 0; l < sweeps / 2 && !rc; ++l) {
-            rc = launch_fused_multi(root, v, fs, n, fs_blocks);
-            if (!rc) rc = launch_fused_multi(root, v, fs + n, n, fs_blocks);
-        }
+        rc = sweep_batch(root, fs, fs + n, n, fs_blocks, count);
         (void)hipEventRecord(e1, root);
         if (hipEventSynchronize(e1) != hipSuccess) rc = BLZ_E_HIP;
         float ms = 0.0f;
         (void)hipEventElapsedTime(&ms, e0, e1);
-        tune_ms[c] = ms / (float)sweeps;
+        ms /= (float)count;
+        if (c < NTUNE) tune_ms[c] = ms;
         if (ms < bestms) {
             bestms = ms;
             bestv = v;
@@ -950,7 +954,8 @@ int blz_batch_set_variant(blz_batch* b, int variant) {
         return BLZ_E_INVALID;
     }
     const int* end = blz::kVariants + blz::NTUNE;
-    if (std::find(blz::kVariants, end, variant) == end) {
+    if (std::find(blz::kVariants, end, variant) == end &&
+        !(variant == blz::VARIANT_TILES && blz::tiles_fit(b->b.every))) {
         blz::set_error("blz_batch_set_variant: not a batch sweep variant (see blz_batch_stats.tune_variant)");
         return BLZ_E_INVALID;
     }

@@ -293,7 +293,9 @@ void clear_step_stats(blz_stats& st) {
 // pressure set to 1.0 (the pressure is restored afterwards; all variants
 // give the same bits); *best = the fastest. Synchronises the stream.
 int Solver::autotune(int sweeps, int* best, float* ms_per_sweep) {
-    static const int cand[] = {2, 4, 8, 102, 103, 202, 203, 402, 403, 1103, 1104, 1105, 1106, 1203, 1204, 1403, 1404};
+    // the one-sweep variants (reported), then several sweeps per launch
+    static const int cand[] = {2,    4,    8,    102,  103,  202,  203,  402,  403,
+                               1103, 1104, 1105, 1106, 1203, 1204, 1403, 1404, VARIANT_TILES};
     sweeps = std::max(2, sweeps & ~1);
     const float dt = s.dt;
     if (tmp_floats < 2 * Np) {
@@ -326,7 +328,7 @@ int Solver::autotune(int sweeps, int* best, float* ms_per_sweep) {
         float ms = 0.0f;
         (void)hipEventElapsedTime(&ms, e0, e1);
         ms /= (float)sweeps;
-        if (ms_per_sweep) ms_per_sweep[k] = ms;
+        if (ms_per_sweep && v != VARIANT_TILES) ms_per_sweep[k] = ms;
         ++k;
         if (ms < bestms) {
             bestms = ms;
@@ -358,9 +360,13 @@ int Solver::autotune(int sweeps, int* best, float* ms_per_sweep) {
 // its result after the step.
 int Solver::project_solve(float dt_) {
     const int cap = s.max_iter_solve;
-    // variant 0: the autotuner's choice for this grid, made at the first solve
-    if (rbgs_variant == 0 && rbgs_auto == 0 && cap > 0)
-        if (int e = autotune(10, &rbgs_auto, nullptr)) return e;
+    // variant 0: several sweeps per launch (faster than every one-sweep
+    // variant on all grids measured, 32^3 .. 256^3); without spare planes
+    // the autotuner's choice for this grid, made at the first solve
+    if (rbgs_variant == 0 && rbgs_auto == 0 && cap > 0) {
+        if (fused_available(*this)) rbgs_auto = VARIANT_TILES;
+        else if (int e = autotune(10, &rbgs_auto, nullptr)) return e;
+    }
     const int q = (int)solves.size();
     if (q >= MAX_SOLVES) {
         set_error("too many pressure solves enqueued without synchronisation");

@@ -1482,10 +1482,11 @@ bool fused_available(const Solver& s) { return s.prb_floats >= 6 * s.Np; }
 // sweep with that many slab groups in flight; 100*w + g (w = 1, 2, 4 waves
 // per block, g = 2, 3 groups in flight) = fused sweeps in pairs, an odd
 // last sweep as two colour passes; 1000 + 100*w + g (g = 3..6) = the same
-// with the row-pair fused sweep; 0 = the autotuner's choice (8 where it
-// has not run).
+// with the row-pair fused sweep; VARIANT_TILES = several sweeps per launch;
+// 0 = VARIANT_TILES, or the autotuner's choice where the spare planes do not
+// exist (8 where it has not run).
 bool rbgs_variant_valid(int v) {
-    return v == 0 || v == 2 || v == 4 || v == 8 || v == 102 || v == 103 || v == 202 || v == 203 || v == 402 ||
+    return v == 0 || v == VARIANT_TILES || v == 2 || v == 4 || v == 8 || v == 102 || v == 103 || v == 202 || v == 203 || v == 402 ||
            v == 403 || v == 1103 || v == 1104 || v == 1105 || v == 1106 || v == 1203 || v == 1204 || v == 1403 ||
            v == 1404;
 }
@@ -1509,6 +1510,39 @@ static int fused_dispatch(Solver& s, int v, float scale, int pairs, const int* s
     }
 }
 
+FusedScene sweep_scene(const Solver& s, float dt, int src, int dst, const int* stop) {
+    const unsigned pb = (unsigned)(s.Np * 4);
+    FusedScene e{};
+    e.base = s.prb;
+    e.nbytes = (unsigned)(s.prb_floats * 4);
+    e.srcR = (unsigned)src * pb;
+    e.srcB = (unsigned)(src + 1) * pb;
+    e.rhsR = 2u * pb;
+    e.rhsB = 3u * pb;
+    e.dstR = (unsigned)dst * pb;
+    e.dstB = (unsigned)(dst + 1) * pb;
+    e.W = s.W;
+    e.H = s.H;
+    e.D = s.D;
+    e.Wp = s.L.Wp;
+    e.Hp = s.L.Hp;
+    e.scale = (s.s.density * s.dx * s.dx) / dt; // gs_solve_kernel :530
+    e.stop = stop;
+    return e;
+}
+
+// the sweeps of VARIANT_TILES on the planes home (through the spare ones),
+// the few left over as colour passes
+static int tile_dispatch(Solver& s, float dt, int sweeps, const int* stop, int home, int* launches) {
+    const int f = tile_family(s.W, s.H);
+    const FusedScene to = sweep_scene(s, dt, home, 4, stop), back = sweep_scene(s, dt, 4, home, stop);
+    int left = 0;
+    if (int e = launch_tile_sweeps(s.stream, f, &to, &back, 0, tile_count(f, s.W, s.H), sweeps, launches, &left))
+        return e;
+    *launches += 2 * left;
+    return left ? rbgs_passes<8>(s, to.scale, left, stop, home) : BLZ_OK;
+}
+
 // `sweeps` sweeps on the judge's pressure planes (the warm start's
 // uncorrected path; same operations as on the home planes): with judge
 // planes of their own, the chosen fused variant in pairs through the spare
@@ -1517,6 +1551,10 @@ static int fused_dispatch(Solver& s, int v, float scale, int pairs, const int* s
 int launch_rbgs_spare(Solver& s, float dt, int sweeps, const int* stop) {
     const float scale = (s.s.density * s.dx * s.dx) / dt;
     const int v = s.rbgs_variant ? s.rbgs_variant : s.rbgs_auto;
+    if (s.judge_set == 6 && v == VARIANT_TILES) {
+        int launches = 0;
+        return tile_dispatch(s, dt, sweeps, stop, 6, &launches);
+    }
     if (s.judge_set == 6 && v >= 100) {
         if (int e = fused_dispatch(s, v, scale, sweeps / 2, stop, 6)) return e;
         return (sweeps & 1) ? rbgs_passes<8>(s, scale, 1, stop, 6) : BLZ_OK;
@@ -1529,6 +1567,10 @@ int launch_rbgs_sweeps(Solver& s, float dt, int sweeps, const int* stop, int* la
     int v = s.rbgs_variant ? s.rbgs_variant : s.rbgs_auto;
     if (v == 0) v = 8;
     if (v >= 100 && !fused_available(s)) v = 8;
+    if (v == VARIANT_TILES) {
+        *kind = 4;
+        return tile_dispatch(s, dt, sweeps, stop, 0, launches);
+    }
     if (v >= 100) {
         const int pairs = sweeps / 2;
         *launches = 2 * pairs + 2 * (sweeps & 1);

@@ -223,8 +223,8 @@ struct Solver {
     std::vector<hipEvent_t> evpool;
     size_t ev_used = 0;
     std::vector<Span> spans;
-    int rbgs_variant = 0; // requested variant (0 = autotuned)
-    int rbgs_auto = 0;    // autotuned variant when rbgs_variant == 0
+    int rbgs_variant = 0; // requested variant (0 = VARIANT_TILES, or autotuned without spare planes)
+    int rbgs_auto = 0;    // the variant used when rbgs_variant == 0
     // learned warm start (attached network; activations of its own)
     const Net* ws_src = nullptr;
     Net* ws_net = nullptr;     // view: shares ws_src's weights, owns activations
@@ -270,9 +270,20 @@ void noise_offsets(const Solver& s, float time, float out[2]);
 int launch_turbulence(Solver& s, float time, float dt);
 int launch_divergence(Solver& s);
 // enqueues `sweeps` sweeps; *launches = kernels launched, *kind = 1 (two
-// colour passes per sweep) or 2 (fused sweeps)
+// colour passes per sweep), 2 (fused sweeps), 3 (row-pair fused sweeps) or 4
+// (several sweeps per launch)
 int launch_rbgs_sweeps(Solver& s, float dt, int sweeps, const int* stop, int* launches, int* kind);
 bool fused_available(const Solver& s);
+// several sweeps per launch (k_sweep.hip): the tile family for a slab, its
+// tiles, and the launches of `sweeps` sweeps
+constexpr int VARIANT_TILES = 2000; // rbgs_variant: these sweeps
+constexpr int TILE_FAMILIES = 4;
+int tile_family(int W, int H);
+int tile_count(int family, int W, int H);
+int launch_tile_sweeps(hipStream_t st, int family, const FusedScene* a, const FusedScene* b, int na, int blocks,
+                       int sweeps, int* launches, int* left);
+// grid s in a sweep table: pressure planes src -> dst (the first plane of each pair)
+FusedScene sweep_scene(const Solver& s, float dt, int src, int dst, const int* stop);
 bool rbgs_variant_valid(int v);
 void clear_step_stats(blz_stats& st);
 int launch_residual_check(Solver& s, float dt, SolveCtl* c, int* host_done, int seq, double tol, int cap, int add,

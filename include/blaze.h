@@ -133,7 +133,8 @@ typedef struct blz_stats {
     int rbgs_launches;        /* RBGS kernel launches behind rbgs_kernel_ms */
     int residual_checks;      /* FP64 residual evaluations in the last step */
     int rbgs_sweeps_timed;    /* RBGS sweeps behind rbgs_kernel_ms */
-    int rbgs_kernel;          /* kernel of the last sweeps: 1 two colour passes, 2 fused sweep, 3 row-pair fused sweep */
+    int rbgs_kernel;          /* kernel of the last sweeps: 1 two colour passes, 2 fused sweep, 3 row-pair fused sweep,
+                                 4 several sweeps per launch */
     int rbgs_sweeps_executed; /* sweeps run in the last step, including the warm start judge's batches on the
                                  path not kept (rbgs_iters counts each judged batch once) */
 } blz_stats;
@@ -200,13 +201,15 @@ int blz_set_timing(blz_solver* h, int on);
    sweeps in pairs through a spare plane set, with 1/2/4 waves per block for
    x = 1/2/4 in 10x; 1x03 .. 1x06 = row-pair fused whole-sweep kernel (two
    rows per wave, 3 to 6 groups in flight, x = 1/2/4 waves per block);
-   0 = default: the autotuner's choice for this grid, made at the first
-   solve (every variant gives the same bits). */
+   2000 = several sweeps per launch, tiles of columns chosen by the grid;
+   0 = default: 2000, or on grids too large for its spare planes the
+   autotuner's choice, made at the first solve (every variant gives the same
+   bits). */
 int blz_set_rbgs_variant(blz_solver* h, int variant);
 /* Autotuner (no reference counterpart): time `sweeps` sweeps of every
    variant above on this grid (pressure restored afterwards) and keep the
-   fastest; ms_per_sweep (optional, 17 entries) receives each time in the
-   order 2, 4, 8, 102, 103, 202, 203, 402, 403, 1103, 1104, 1105, 1106,
+   fastest; ms_per_sweep (optional, 17 entries) receives the time of each
+   but 2000, in the order 2, 4, 8, 102, 103, 202, 203, 402, 403, 1103, 1104, 1105, 1106,
    1203, 1204, 1403, 1404 (fused ones skipped when the spare planes do not
    exist). */
 int blz_autotune_rbgs(blz_solver* h, int sweeps, int* variant, float* ms_per_sweep);
@@ -383,12 +386,14 @@ int blz_batch_destroy(blz_batch* b);
 /* Borrowed handle of scene i (sourcing, fields, stats); do not destroy. */
 int blz_batch_solver(blz_batch* b, int i, blz_solver** out);
 int blz_batch_set_warm_start(blz_batch* b, blz_net* net);
-/* Time `sweeps` sweeps of each candidate tile configuration (slab groups in
-   flight x waves per block) over the whole batch, keep the fastest; the
-   pressure fields are restored afterwards. */
+/* Time `sweeps` sweeps of each candidate (slab groups in flight x waves per
+   block, and variant 2000 of blz_set_rbgs_variant where
+   residual_check_every is at least 4) over the whole batch, keep the
+   fastest; the pressure fields are restored afterwards. Without it the batch
+   sweeps with variant 2000 where that fits, else 103. */
 int blz_batch_autotune(blz_batch* b, int sweeps, int* variant);
-/* Use one of the autotuner's candidates (blz_batch_stats.tune_variant) for
-   the batch's sweeps (no reference counterpart; every candidate gives the
+/* Use one of the autotuner's candidates (blz_batch_stats.tune_variant, or
+   2000) for the batch's sweeps (no reference counterpart; every candidate gives the
    same bits). */
 int blz_batch_set_variant(blz_batch* b, int variant);
 int blz_batch_step(blz_batch* b, float time);

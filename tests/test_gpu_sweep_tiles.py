@@ -1,0 +1,87 @@
+"""Several sweeps per launch (the default sweeps, variant 2000) against the
+oracle bit for bit: every tile size the grid can get, one-column and clipped
+tiles at both rims, one to many slab groups (partly filled last groups), and
+sweep counts that leave one to three sweeps to the colour passes."""
+import numpy as np
+import pytest
+
+B = pytest.importorskip("blaze_amd")
+O = pytest.importorskip("oracle")
+from helpers import compare, random_state, settings  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+# 4x4 tiles up to 64x64 columns, then 8x4, 8x8 and 16x16
+SHAPES = [(4, 4, 4), (6, 5, 9), (34, 33, 32), (64, 61, 6), (66, 90, 13), (90, 75, 5), (130, 66, 22), (122, 128, 8),
+          (162, 133, 7), (200, 98, 18)]
+
+
+def pair(s, st):
+    g, o = B.Solver(s), O.Oracle(s)
+    for w, a in st.items():
+        g.set_field(w, a)
+        o.set_field(w, a)
+    return g, o
+
+
+@pytest.mark.parametrize("res", SHAPES, ids=["x".join(map(str, r)) for r in SHAPES])
+@pytest.mark.parametrize("iters", [3, 5, 7, 10, 22])
+def test_tile_sweeps_bitwise(res, iters):
+    print(f"[tiles] res={res} iters={iters}", flush=True)
+    s = settings(B, res, max_iter_solve=iters)
+    g, o = pair(s, random_state(s, seed=iters + sum(res)))
+    for x in (g, o):
+        x.run_stage(B.STAGE_PRESSURE, 0.0, 1.0 / 24.0)
+    compare("tile sweeps", g.field(B.FIELD_P), o.field(B.FIELD_P))
+    assert g.stats().rbgs_kernel == 4
+
+
+@pytest.mark.parametrize("kind", ["tiny", "negzero", "decay", "inf"])
+@pytest.mark.parametrize("res", [(40, 36, 24), (90, 75, 10), (162, 133, 9)], ids=["4x4", "8x4", "16x16"])
+def test_tile_sweeps_exact_division(kind, res):
+    """Numerators outside the fast division's range in some lanes, groups or
+    slabs only, and an infinity that spreads."""
+    print(f"[tiles-exact] {kind} res={res}", flush=True)
+    s = settings(B, res, max_iter_solve=10)
+    st = random_state(s, seed=3)
+    p, r = st[B.FIELD_P], st[B.FIELD_RHS]
+    if kind == "tiny":
+        st[B.FIELD_P], st[B.FIELD_RHS] = p * np.float32(1e-38), r * np.float32(3e-38)
+    elif kind == "negzero":
+        st[B.FIELD_P], st[B.FIELD_RHS] = np.full_like(p, -0.0), np.full_like(r, -0.0)
+        st[B.FIELD_RHS][3, 5, 7] = np.float32(1e-3)
+    elif kind == "decay":
+        st[B.FIELD_P], st[B.FIELD_RHS] = np.zeros_like(p), np.zeros_like(r)
+        st[B.FIELD_RHS][1, 20, 21] = np.float32(1e-30)
+    else:
+        st[B.FIELD_P][4, 9, 11] = np.float32(np.inf)
+    g, o = pair(s, st)
+    for x in (g, o):
+        x.run_stage(B.STAGE_PRESSURE, 0.0, 1.0 / 24.0)
+    compare(f"tile sweeps {kind}", g.field(B.FIELD_P), o.field(B.FIELD_P))
+
+
+@pytest.mark.parametrize("sizes", [((32, 24, 20), (16, 40, 9)), ((96, 88, 12), (130, 66, 7)),
+                                   ((162, 133, 8), (34, 36, 16))], ids=["small", "middle", "large"])
+def test_batch_tile_sweeps_equal_single_scenes(sizes):
+    """Scenes of unlike sizes share a tile in the batch and each get what
+    they get alone; the variant can be set by its number."""
+    print(f"[tiles-batch] {sizes}", flush=True)
+    sets = [settings(B, r, max_iter_solve=30, residual_tol=1e-6, residual_check_every=10, buoyancy=1.0, gravity=-9.8)
+            for r in sizes]
+    b = B.Batch(sets)
+    assert b.stats().variant == 2000
+    b.set_variant(2000)
+    states = [random_state(s, seed=q, vel_scale=0.5) for q, s in enumerate(sets)]
+    single = [B.Solver(s) for s in sets]
+    for q, st in enumerate(states):
+        for w, a in st.items():
+            b.scenes[q].set_field(w, a)
+            single[q].set_field(w, a)
+    for _ in range(2):
+        b.step(0.0)
+        for g in single:
+            g.step(0.0)
+    for q, g in enumerate(single):
+        for w in (B.FIELD_T, B.FIELD_U, B.FIELD_V, B.FIELD_W, B.FIELD_P):
+            compare(f"scene {q} field {w}", b.scenes[q].field(w), g.field(w))
