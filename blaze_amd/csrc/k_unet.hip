@@ -17,7 +17,6 @@ namespace blz {
 
 namespace {
 
-typedef short s4v __attribute__((ext_vector_type(4)));
 typedef short s8v __attribute__((ext_vector_type(8)));
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 typedef float f4m __attribute__((ext_vector_type(4)));
@@ -251,70 +250,167 @@ __global__ void __launch_bounds__(256) k_conv3_multi(const MView* __restrict__ t
                             blockIdx.x);
 }
 
-// weight gradient: dW[tap][co][ci] += sum_v G[v][co] X[v+tap][ci]. A wave owns
-// one 16x16 (co, ci) tile and a run of voxels; per 16 voxels the G fragment
-// (A = 16 co x 16 voxels) is loaded once and used for all 27 taps (B = 16
-// voxels x 16 ci, shifted by the tap). FP32 partial tiles are added with
-// atomics.
-__global__ void __launch_bounds__(256) k_conv3_dw(const bf16* __restrict__ X, int Cx, int xoff, int Cin,
-                                                  const bf16* __restrict__ Gd, int Cg, int goff, int Cout,
-                                                  float* __restrict__ dW, Geo g, long long nvox, long long run) {
-    const int lane = threadIdx.x & 63;
-    const long long wv = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int nct = Cout >> 4, ncit = Cin >> 4;
-    const int tiles = nct * ncit;
-    const long long chunk = wv / tiles;
-    const int tile = (int)(wv % tiles);
-    const int cot = tile / ncit, cit = tile % ncit;
-    const long long vbeg = chunk * run;
-    if (vbeg >= nvox) return;
-    const long long vend = min(nvox, vbeg + run);
+// ---- weight gradient: dW[tap][co][ci] = sum_v G[v][co] X[v+tap][ci] ----
+// A product over the voxels, which channels-last activations hold strided.
+// So both operands are first copied channel by channel with zero padding
+// (k_dw_rows): rows of Wp = W + 1 rounded up to 8 elements, each plane
+// preceded by a zero row and each volume by a zero plane. In that order a tap
+// is one constant shift, dz plane + dy Wp + dx, which meets zeros wherever it
+// leaves the grid, the sum runs over one contiguous range (padding included:
+// 1.33 of the voxels at 32^3), and eight voxels of a channel are one 16-byte
+// load. The eight of the taps dx = -1 and +1 come from the eight of dx = 0 and
+// the two elements beside them by funnel shifts. (An infinite activation
+// next to padding gives NaN where skipping the pair would give infinity.)
+//
+// A wave owns one 16x16 (co, ci) tile for all 27 taps and a run of 32-element
+// chunks (A: 16 co x 32, B: 32 x 16 ci of v_mfma_f32_16x16x32_bf16); the four
+// waves of a workgroup add their tiles through LDS, the workgroups' tiles go
+// to a buffer that k_dw_sum adds up in a fixed order: no atomics, every run
+// gives the same bits. Bound by the operands' L1 loads (28 per 27 MFMAs).
+// A training step at 8 x 32^3 runs ten of these (0.37 ms, with the copies and
+// sums 0.54 of 1.34 ms). Gathering every operand element by itself (2-byte
+// loads, 108 per 16 voxels) with atomic sums took 26.4 of 27.8 ms.
+constexpr int DW_RUN = 128; // elements that one workgroup of k_dw_rows copies
+struct DwGeo {
+    int B, D, H, W, Wp;
+    int lead;          // zero rows before the first volume (a plane and a row, and one for the shift by -1)
+    long long rows;    // rows of the volumes, zero rows between them included
+    long long stride;  // elements per channel, the zero rows around and 64 more included
+};
+DwGeo dw_geo(const Geo& g) {
+    DwGeo d{g.B, g.D, g.H, g.W, (g.W + 8) / 8 * 8, g.H + 3, (long long)g.B * (g.D + 1) * (g.H + 1), 0};
+    d.stride = ((d.rows + 2 * d.lead) * d.Wp + 64 + DW_RUN - 1) / DW_RUN * DW_RUN;
+    return d;
+}
+
+// DW_RUN elements of the padded order of all C channels of a view per
+// workgroup, transposed through LDS (the padded order has fewer than 2^31
+// elements: nv C does, for the layers' C >= 16). Bound by its memory traffic.
+__global__ void __launch_bounds__(256) k_dw_rows(const bf16* __restrict__ X, int Cx, int xoff, int C, DwGeo d,
+                                                 bf16* __restrict__ out) {
+    constexpr int PITCH = DW_RUN + 8; // 16-byte rows
+    __shared__ bf16 sm[96 * PITCH];
+    const unsigned e0 = blockIdx.x * DW_RUN, c8 = (unsigned)C / 8, lead = (unsigned)(d.lead * d.Wp);
+    for (unsigned t = threadIdx.x; t < DW_RUN * c8; t += 256) {
+        const unsigned k = t / c8, c = (t - k * c8) * 8;
+        const unsigned e = e0 + k - lead; // wraps before the first volume
+        s8v q = {0, 0, 0, 0, 0, 0, 0, 0};
+        const unsigned r = e / (unsigned)d.Wp, x = e - r * d.Wp; // row of the volumes, place in it
+        if (e < 0x80000000u && r < (unsigned)d.rows && x < (unsigned)d.W) {
+            const unsigned p = r / (unsigned)(d.H + 1), yy = r - p * (d.H + 1);
+            const unsigned b = p / (unsigned)(d.D + 1), zz = p - b * (d.D + 1);
+            if (yy && zz) {
+                const long long v = (((long long)b * d.D + zz - 1) * d.H + yy - 1) * d.W + x;
+                q = *(const s8v*)(X + v * Cx + xoff + c);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sm[(c + j) * PITCH + k] = (bf16)q[j];
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < C * (DW_RUN / 8); t += 256) {
+        const int c = t / (DW_RUN / 8), x = t % (DW_RUN / 8) * 8;
+        *(s8v*)(out + c * d.stride + e0 + x) = *(const s8v*)(sm + c * PITCH + x);
+    }
+}
+
+typedef unsigned u4b __attribute__((ext_vector_type(4)));
+
+// chunks [w per, (w + 1) per) of wave w = 4 blockIdx.x + its place in the
+// workgroup; part[blockIdx.x][tile][tap][lane][4]
+__global__ void __launch_bounds__(256) k_conv3_dw(const bf16* __restrict__ Xt, const bf16* __restrict__ Gt, DwGeo d,
+                                                  int ncit, long long nchunk, int per, float* __restrict__ part) {
+    __shared__ f4m sm[27 * 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int li = lane & 15, kb = lane >> 4;
-    const long long HW = (long long)g.H * g.W;
+    const int cot = blockIdx.y / ncit, cit = blockIdx.y % ncit;
+    const long long plane = (long long)(d.H + 1) * d.Wp;
+    const long long c0 = ((long long)blockIdx.x * 4 + w) * per, c1 = min(nchunk, c0 + per);
+    const long long first = (long long)d.lead * d.Wp + c0 * 32 + 8 * kb;
+    const bf16* ga = Gt + (cot * 16 + li) * d.stride + first;
+    const bf16* xa = Xt + (cit * 16 + li) * d.stride + first;
     f4m acc[27];
 #pragma unroll
     for (int t = 0; t < 27; ++t) acc[t] = f4m{0.f, 0.f, 0.f, 0.f};
-    for (long long vb = vbeg; vb < vend; vb += 16) {
-        s4v a;
-        int bq[4], zq[4], yq[4], xq[4];
-        bool okq[4];
+    for (long long c = c0; c < c1; ++c, ga += 32, xa += 32) {
+        const bf8v a = *(const bf8v*)ga;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const long long v = vb + kb * 4 + q;
-            okq[q] = v < vend;
-            vox_coords(okq[q] ? v : vbeg, g, bq[q], zq[q], yq[q], xq[q]);
-            a[q] = okq[q] ? (short)Gd[v * Cg + goff + cot * 16 + li] : (short)0;
-        }
-#pragma unroll
-        for (int tap = 0; tap < 27; ++tap) {
-            const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-            s4v bx;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int zz = zq[q] + dz, yy = yq[q] + dy, xx = xq[q] + dx;
-                const bool inb = okq[q] && zz >= 0 && zz < g.D && yy >= 0 && yy < g.H && xx >= 0 && xx < g.W;
-                const long long vv = vb + kb * 4 + q + dz * HW + dy * g.W + dx;
-                bx[q] = inb ? (short)X[vv * Cx + xoff + cit * 16 + li] : (short)0;
-            }
-            acc[tap] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bx, acc[tap], 0, 0, 0);
+        for (int row = 0; row < 9; ++row) {
+            const bf16* q = xa + (row / 3 - 1) * plane + (row % 3 - 1) * d.Wp;
+            const u4b v = *(const u4b*)q;
+            const unsigned lo = *(const unsigned*)(q - 2), hi = *(const unsigned*)(q + 8);
+            const unsigned m0 = __builtin_amdgcn_alignbit(v[0], lo, 16), m1 = __builtin_amdgcn_alignbit(v[1], v[0], 16),
+                           m2 = __builtin_amdgcn_alignbit(v[2], v[1], 16), m3 = __builtin_amdgcn_alignbit(v[3], v[2], 16),
+                           m4 = __builtin_amdgcn_alignbit(hi, v[3], 16);
+            const u4b l = {m0, m1, m2, m3}, r = {m1, m2, m3, m4};
+            acc[3 * row] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf8v, l), acc[3 * row], 0, 0, 0);
+            acc[3 * row + 1] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf8v, v), acc[3 * row + 1], 0, 0, 0);
+            acc[3 * row + 2] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf8v, r), acc[3 * row + 2], 0, 0, 0);
         }
     }
-    // D[i][j]: i = co (4*kb + q), j = ci (li)
+    // the waves' tiles, added in wave order
+    for (int k = 0; k < 4; ++k) {
+        if (w == k) {
 #pragma unroll
-    for (int tap = 0; tap < 27; ++tap)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            atomicAdd(&dW[((size_t)tap * Cout + cot * 16 + kb * 4 + q) * Cin + cit * 16 + li], acc[tap][q]);
+            for (int t = 0; t < 27; ++t) {
+                const f4m s = k ? sm[t * 64 + lane] + acc[t] : acc[t];
+                if (k < 3) sm[t * 64 + lane] = s;
+                else
+                    *(f4m*)(part + (((size_t)blockIdx.x * gridDim.y + blockIdx.y) * 27 + t) * 256 + lane * 4) = s;
+            }
+        }
+        __syncthreads();
+    }
 }
 
-// Wt[tap'][ci][co] = W[26 - tap'][co][ci]: the input gradient is the forward
-// convolution of the output gradient with these weights
-__global__ void k_wflip(const bf16* __restrict__ W, bf16* __restrict__ Wt, int Cout, int Cin) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int n = 27 * Cout * Cin;
+// dW of one layer: the workgroups' tiles added, every 16th by one wave, then
+// the waves' sums in order. D[i][j] of a tile: i = co (4 (lane / 16) + q),
+// j = ci (lane % 16)
+__global__ void __launch_bounds__(1024) k_dw_sum(const float* __restrict__ part, int splits, int ncit, int Cout,
+                                                 int Cin, float* __restrict__ dW) {
+    __shared__ f4m sm[16 * 64];
+    const int tile = blockIdx.y, tap = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const size_t step = (size_t)gridDim.y * 27 * 64;
+    const f4m* p = (const f4m*)part + ((size_t)tile * 27 + tap) * 64 + lane;
+    f4m s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int k = w; k < splits; k += 16) s += p[k * step];
+    sm[w * 64 + lane] = s;
+    __syncthreads();
+    if (threadIdx.x >= 256) return;
+    const int e = threadIdx.x;
+    float v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) v += ((const float*)sm)[k * 256 + e];
+    const int l = e >> 2, co = (tile / ncit) * 16 + 4 * (l >> 4) + (e & 3), ci = (tile % ncit) * 16 + (l & 15);
+    dW[((size_t)tap * Cout + co) * Cin + ci] = v;
+}
+
+// BF16 weights, as they are (Wb) and flipped and transposed (Wt[tap'][ci][co]
+// = W[26 - tap'][co][ci]: the input gradient is the forward convolution of
+// the output gradient with these), of all layers in one launch
+struct Layers {
+    int off[L_NCONV + 1], cin[L_NCONV], cout[L_NCONV];
+};
+__global__ void __launch_bounds__(256) k_weights(const float* __restrict__ P, bf16* __restrict__ Wb,
+                                                 bf16* __restrict__ Wt, Layers L, int n) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
     if (t >= n) return;
-    const int ci = t % Cin, co = (t / Cin) % Cout, tap = t / (Cin * Cout);
-    Wt[((size_t)(26 - tap) * Cin + ci) * Cout + co] = W[t];
+    const bf16 w = f2bf(P[t]);
+    Wb[t] = w;
+    if (t >= L.off[L_NCONV]) return;
+    int l = 0;
+#pragma unroll
+    for (int q = 1; q < L_NCONV; ++q)
+        if (t >= L.off[q]) l = q;
+    int o = 0, cin = 0, cout = 0;
+#pragma unroll
+    for (int q = 0; q < L_NCONV; ++q)
+        if (q == l) o = L.off[q], cin = L.cin[q], cout = L.cout[q];
+    const int r = t - o, ci = r % cin, co = (r / cin) % cout, tap = r / (cin * cout);
+    Wt[o + ((26 - tap) * cin + ci) * cout + co] = w;
 }
 
 __device__ __forceinline__ long long parent_of(long long v, const Geo& fine, int& b, int& z, int& y, int& x) {
@@ -433,44 +529,79 @@ __global__ void __launch_bounds__(256) k_mse(const float* __restrict__ out, cons
     if (threadIdx.x == 0) atomicAdd(loss, (sm[0] + sm[1] + sm[2] + sm[3]) / (double)n);
 }
 
-// head backward: gX[v][c] = gout[v] w[c] (ReLU mask of X), gw[c] += sum_v gout[v] X[v][c]
+// head backward: gX[v][c] = gout[v] w[c] (ReLU mask of X), and each
+// workgroup's part of gw[c] = sum_v gout[v] X[v][c] (added up in order by
+// k_head_sum: 32768 atomic adds to 16 floats took 0.43 ms at 8 x 32^3)
 __global__ void __launch_bounds__(256) k_head_bwd(const float* __restrict__ gout, const bf16* __restrict__ X,
                                                   const float* __restrict__ w, bf16* __restrict__ gX,
-                                                  float* __restrict__ gw, long long n) {
-    float acc[NET_HEAD];
+                                                  float* __restrict__ part, long long n) {
+    float acc[NET_HEAD], wb[NET_HEAD];
 #pragma unroll
-    for (int c = 0; c < NET_HEAD; ++c) acc[c] = 0.0f;
+    for (int c = 0; c < NET_HEAD; ++c) {
+        acc[c] = 0.0f;
+        wb[c] = bf2f(f2bf(w[c]));
+    }
     for (long long v = (long long)blockIdx.x * 256 + threadIdx.x; v < n; v += (long long)gridDim.x * 256) {
         const float go = gout[v];
 #pragma unroll
-        for (int c = 0; c < NET_HEAD; ++c) {
-            const float xv = bf2f(X[v * NET_HEAD + c]);
-            acc[c] = fmaf(go, xv, acc[c]);
-            const float gx = go * bf2f(f2bf(w[c]));
-            gX[v * NET_HEAD + c] = f2bf(xv > 0.0f ? gx : NET_LEAK * gx);
+        for (int h = 0; h < NET_HEAD / 8; ++h) {
+            const s8v xv = *(const s8v*)(X + v * NET_HEAD + 8 * h);
+            s8v gv;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int c = 8 * h + k;
+                const float x = bf2f((bf16)xv[k]);
+                acc[c] = fmaf(go, x, acc[c]);
+                const float gx = go * wb[c];
+                gv[k] = (short)f2bf(x > 0.0f ? gx : NET_LEAK * gx);
+            }
+            *(s8v*)(gX + v * NET_HEAD + 8 * h) = gv;
         }
     }
+    __shared__ float sm[4][NET_HEAD];
 #pragma unroll
     for (int c = 0; c < NET_HEAD; ++c) {
         float s = acc[c];
         for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
-        if ((threadIdx.x & 63) == 0) atomicAdd(&gw[c], s);
+        if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6][c] = s;
     }
+    __syncthreads();
+    if (threadIdx.x < NET_HEAD)
+        part[blockIdx.x * NET_HEAD + threadIdx.x] =
+            ((sm[0][threadIdx.x] + sm[1][threadIdx.x]) + sm[2][threadIdx.x]) + sm[3][threadIdx.x];
 }
 
-// global gradient-norm clipping: *scale = min(1, maxnorm / ||G||) (one block)
-__global__ void __launch_bounds__(1024) k_gclip(const float* __restrict__ G, size_t n, float maxnorm,
-                                                float* __restrict__ scale) {
+// gw[c]: one wave per channel adds every 64th part, then its lanes' sums
+__global__ void __launch_bounds__(1024) k_head_sum(const float* __restrict__ part, int n, float* __restrict__ gw) {
+    const int c = threadIdx.x >> 6, l = threadIdx.x & 63;
+    float s = 0.0f;
+    for (int q = l; q < n; q += 64) s += part[q * NET_HEAD + c];
+    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (l == 0) gw[c] = s;
+}
+
+// global gradient-norm clipping: *scale = min(1, maxnorm / ||G||), from the
+// workgroups' sums of squares
+constexpr int GNORM_BLOCKS = 256, HEAD_BLOCKS = 512;
+__global__ void __launch_bounds__(256) k_gnorm(const float* __restrict__ G, size_t n, double* __restrict__ part) {
     double a = 0.0;
-    for (size_t t = threadIdx.x; t < n; t += 1024) a += (double)G[t] * (double)G[t];
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (size_t)GNORM_BLOCKS * 256)
+        a += (double)G[t] * (double)G[t];
     for (int o = 32; o >= 1; o >>= 1) a += __shfl_xor(a, o, 64);
-    __shared__ double sm[16];
+    __shared__ double sm[4];
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = a;
+    __syncthreads();
+    if (threadIdx.x == 0) part[blockIdx.x] = ((sm[0] + sm[1]) + sm[2]) + sm[3];
+}
+__global__ void __launch_bounds__(GNORM_BLOCKS) k_gclip(const double* __restrict__ part, float maxnorm,
+                                                        float* __restrict__ scale) {
+    double a = part[threadIdx.x];
+    for (int o = 32; o >= 1; o >>= 1) a += __shfl_xor(a, o, 64);
+    __shared__ double sm[4];
     if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = a;
     __syncthreads();
     if (threadIdx.x == 0) {
-        double tot = 0.0;
-        for (int q = 0; q < 16; ++q) tot += sm[q];
-        const double nrm = sqrt(tot);
+        const double nrm = sqrt(((sm[0] + sm[1]) + sm[2]) + sm[3]);
         *scale = (nrm > (double)maxnorm && nrm == nrm) ? (float)((double)maxnorm / nrm) : (nrm == nrm ? 1.0f : 0.0f);
     }
 }
@@ -486,11 +617,6 @@ __global__ void k_adam(float* __restrict__ P, const float* __restrict__ G, float
     M[t] = m;
     V[t] = v;
     P[t] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
-}
-
-__global__ void k_to_bf16(const float* __restrict__ P, bf16* __restrict__ Wb, size_t n) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) Wb[t] = f2bf(P[t]);
 }
 
 __global__ void k_fill_f32(float* __restrict__ p, size_t n, float v) {
@@ -583,18 +709,43 @@ static int conv_fwd(Net& n, int layer, TV x, TV y, TV mask, bool relu, const Net
     return BLZ_OK;
 }
 
+// the weight gradient's launch: 32-element chunks of the padded range, at
+// least 4 per wave, about two workgroups per CU over all tiles
+struct DwPlan {
+    DwGeo d;
+    int tiles, per, splits;
+    long long nchunk;
+    size_t xbytes, gbytes, pbytes; // workspace: the copies of X and G, the tiles' parts
+};
+static DwPlan dw_plan(int layer, const NetDims& d) {
+    DwPlan p;
+    const int cin = kConv[layer].cin, cout = kConv[layer].cout;
+    p.d = dw_geo(Geo{d.B, d.D, d.H, d.W});
+    p.tiles = (cout / 16) * (cin / 16);
+    p.nchunk = (p.d.rows * p.d.Wp + 31) / 32;
+    const long long want = std::max(1, 512 / p.tiles);
+    p.per = (int)std::max<long long>(4, (p.nchunk + 4 * want - 1) / (4 * want));
+    p.splits = (int)((p.nchunk + 4ll * p.per - 1) / (4ll * p.per));
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    p.xbytes = up((size_t)cin * p.d.stride * 2);
+    p.gbytes = up((size_t)cout * p.d.stride * 2);
+    p.pbytes = up((size_t)p.splits * p.tiles * 27 * 256 * 4);
+    return p;
+}
+
 static int conv_dw(Net& n, int layer, TV x, TV gy, const NetDims& d) {
     const int cin = kConv[layer].cin, cout = kConv[layer].cout;
-    const Geo g{d.B, d.D, d.H, d.W};
-    const long long nv = d.n();
-    const int tiles = (cout / 16) * (cin / 16);
-    // voxel run per wave: at least 512, at most 32 runs per tile
-    long long run = std::max<long long>(512, (nv + 31) / 32);
-    run = (run + 15) / 16 * 16;
-    const long long chunks = (nv + run - 1) / run;
-    const long long waves = chunks * tiles;
-    hipLaunchKernelGGL(k_conv3_dw, dim3(nblk(waves, 4)), dim3(256), 0, n.stream, x.p, x.C, x.off, cin, gy.p, gy.C,
-                       gy.off, cout, n.G + n.off[layer], g, nv, run);
+    const DwPlan p = dw_plan(layer, d);
+    bf16* xt = (bf16*)n.dw_buf;
+    bf16* gt = (bf16*)((char*)n.dw_buf + p.xbytes);
+    float* part = (float*)((char*)n.dw_buf + p.xbytes + p.gbytes);
+    const dim3 rows((unsigned)(p.d.stride / DW_RUN));
+    hipLaunchKernelGGL(k_dw_rows, rows, dim3(256), 0, n.stream, x.p, x.C, x.off, cin, p.d, xt);
+    hipLaunchKernelGGL(k_dw_rows, rows, dim3(256), 0, n.stream, gy.p, gy.C, gy.off, cout, p.d, gt);
+    hipLaunchKernelGGL(k_conv3_dw, dim3((unsigned)p.splits, (unsigned)p.tiles), dim3(256), 0, n.stream, xt, gt, p.d,
+                       cin / 16, p.nchunk, p.per, part);
+    hipLaunchKernelGGL(k_dw_sum, dim3(27, (unsigned)p.tiles), dim3(1024), 0, n.stream, part, p.splits, cin / 16, cout,
+                       cin, n.G + n.off[layer]);
     NET_HIP(hipGetLastError());
     return BLZ_OK;
 }
@@ -608,6 +759,7 @@ Net::~Net() {
         if (stream) (void)hipStreamDestroy(stream);
     }
     if (act) (void)hipFree(act);
+    if (dw_buf) (void)hipFree(dw_buf);
 }
 
 int Net::init_view(const Net& src, hipStream_t st) {
@@ -662,13 +814,37 @@ int Net::init(unsigned long long seed) {
 }
 
 int Net::refresh_weights() {
-    hipLaunchKernelGGL(k_to_bf16, dim3(nblk((long long)nparam, 256)), dim3(256), 0, stream, P, Wb, nparam);
+    Layers L;
     for (int l = 0; l < L_NCONV; ++l) {
-        const int n = 27 * kConv[l].cout * kConv[l].cin;
-        hipLaunchKernelGGL(k_wflip, dim3(nblk(n, 256)), dim3(256), 0, stream, Wb + off[l], Wt + off[l],
-                           kConv[l].cout, kConv[l].cin);
+        L.off[l] = (int)off[l];
+        L.cin[l] = kConv[l].cin;
+        L.cout[l] = kConv[l].cout;
     }
+    L.off[L_NCONV] = (int)off[L_NCONV];
+    hipLaunchKernelGGL(k_weights, dim3(nblk((long long)nparam, 256)), dim3(256), 0, stream, P, Wb, Wt, L, (int)nparam);
     NET_HIP(hipGetLastError());
+    return BLZ_OK;
+}
+
+// scratch of a training step for the current dims: the weight gradients', one
+// layer at a time, and before and after them the head's and the norm's sums
+int Net::ensure_backward() {
+    static constexpr int level[L_NCONV] = {0, 0, 1, 1, 2, 2, 1, 1, 0, 0};
+    const NetDims lv[3] = {dims, dims.half(), dims.half().half()};
+    size_t need = std::max((size_t)HEAD_BLOCKS * NET_HEAD * 4, (size_t)GNORM_BLOCKS * 8);
+    for (int l = 0; l < L_NCONV; ++l) {
+        const DwPlan p = dw_plan(l, lv[level[l]]);
+        need = std::max(need, p.xbytes + p.gbytes + p.pbytes);
+    }
+    if (need <= dw_bytes) return BLZ_OK;
+    if (dw_buf) NET_HIP(hipFree(dw_buf));
+    dw_buf = nullptr;
+    dw_bytes = 0;
+    if (hipMalloc(&dw_buf, need) != hipSuccess) {
+        set_error("hipMalloc failed for the weight gradients' scratch");
+        return BLZ_E_NOMEM;
+    }
+    dw_bytes = need;
     return BLZ_OK;
 }
 
@@ -947,10 +1123,12 @@ int Net::backward() {
     const long long n1 = d1.n(), n2 = d2.n(), n3 = d3.n();
     const TV none{nullptr, 0, 0};
     int e;
-    hipLaunchKernelGGL(k_fill_f32, dim3(nblk((long long)nparam, 256)), dim3(256), 0, stream, G, nparam, 0.0f);
+    if ((e = ensure_backward())) return e;
     // head (ReLU mask of b5 folded in)
-    hipLaunchKernelGGL(k_head_bwd, dim3((unsigned)std::min<long long>(nblk(n1, 256), 512)), dim3(256), 0, stream,
-                       gout, b5, P + off[L_NCONV], g_b5, G + off[L_NCONV], n1);
+    const unsigned hb = (unsigned)std::min<long long>(nblk(n1, 256), HEAD_BLOCKS);
+    hipLaunchKernelGGL(k_head_bwd, dim3(hb), dim3(256), 0, stream, gout, b5, P + off[L_NCONV], g_b5, (float*)dw_buf,
+                       n1);
+    hipLaunchKernelGGL(k_head_sum, dim3(1), dim3(NET_HEAD * 64), 0, stream, (const float*)dw_buf, (int)hb, G + off[L_NCONV]);
     NET_HIP(hipGetLastError());
     // d1b: a5 -> b5
     if ((e = conv_dw(*this, L_D1B, TV{a5, 16, 0}, TV{g_b5, 16, 0}, d1))) return e;
@@ -1001,7 +1179,8 @@ int Net::adam(float lr, float b1, float b2, float eps) {
     ++adam_t;
     const float c1 = 1.0f - std::pow(b1, (float)adam_t), c2 = 1.0f - std::pow(b2, (float)adam_t);
     float* gscale = out + dims.n(); // one float after the prediction (see ensure_dims)
-    hipLaunchKernelGGL(k_gclip, dim3(1), dim3(1024), 0, stream, G, nparam, 1.0f, gscale);
+    hipLaunchKernelGGL(k_gnorm, dim3(GNORM_BLOCKS), dim3(256), 0, stream, G, nparam, (double*)dw_buf);
+    hipLaunchKernelGGL(k_gclip, dim3(1), dim3(GNORM_BLOCKS), 0, stream, (const double*)dw_buf, 1.0f, gscale);
     hipLaunchKernelGGL(k_adam, dim3(nblk((long long)nparam, 256)), dim3(256), 0, stream, P, G, M, V, nparam, lr, b1,
                        b2, eps, c1, c2, gscale);
     NET_HIP(hipGetLastError());

@@ -79,6 +79,9 @@ struct Net {
     double* loss = nullptr;  // device accumulator (sum of squared errors)
     double* loss_host = nullptr;
 
+    void* dw_buf = nullptr; // scratch of the backward pass (ensure_backward)
+    size_t dw_bytes = 0;
+
     bool view = false; // parameters borrowed from another Net
 
     ~Net();
@@ -89,6 +92,7 @@ struct Net {
     int forward();         // x0 -> out (stream-ordered)
     int loss_and_grad();   // out, target -> gout, *loss (mean squared error)
     int backward();        // gout -> G (overwritten)
+    int ensure_backward();
     int adam(float lr, float b1, float b2, float eps);
 };
 
