@@ -71,21 +71,32 @@ inline bool dx_pow2(float dx, float* inv) {
     return std::isfinite(*inv) && *inv * dx == 1.0f;
 }
 
-// Gathers of the samplers below. A field of fewer than 2^29 floats is read
-// with buffer loads: a 32-bit byte offset against a buffer resource built
-// from the field's (uniform) base, so the 64-bit address arithmetic of a
-// pointer gather disappears; the values read are the same. Larger fields
-// take the pointer path (a wave-uniform branch).
+// Gathers of the samplers below, of two or four neighbours along x at a time
+// (any element may come first: the loads need 4-byte alignment). A field of
+// fewer than 2^29 floats is read with buffer loads: a 32-bit byte offset
+// against a buffer resource built from the field's (uniform) base, so the
+// 64-bit address arithmetic of a pointer gather disappears; the values read
+// are the same. Larger fields take the pointer path (a wave-uniform branch).
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2a4 __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
 struct GatherB {
     __amdgpu_buffer_rsrc_t r;
-    __device__ __forceinline__ float operator()(long long idx) const {
-        // the builtin returns the 32 bits as an integer: reinterpret them
-        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)idx * 4, 0, 0));
+    // the builtins return the bits as integers: reinterpret them
+    __device__ __forceinline__ f32x2 two(long long idx) const {
+        return __builtin_bit_cast(f32x2, (u32x2)__builtin_amdgcn_raw_buffer_load_b64(r, (int)idx * 4, 0, 0));
+    }
+    __device__ __forceinline__ f32x4 four(long long idx) const {
+        return __builtin_bit_cast(f32x4, (u32x4)__builtin_amdgcn_raw_buffer_load_b128(r, (int)idx * 4, 0, 0));
     }
 };
 struct GatherP {
     const float* a;
-    __device__ __forceinline__ float operator()(long long idx) const { return a[idx]; }
+    __device__ __forceinline__ f32x2 two(long long idx) const { return *(const f32x2a4*)(a + idx); }
+    __device__ __forceinline__ f32x4 four(long long idx) const { return *(const f32x4a4*)(a + idx); }
 };
 __device__ __forceinline__ bool gather_buffered(const Gv& g) {
     return (long long)g.nx * g.ny * g.nz < (1ll << 29);
@@ -94,7 +105,7 @@ __device__ __forceinline__ GatherB gather_b(const Gv& g) {
     return GatherB{__builtin_amdgcn_make_buffer_rsrc((void*)g.a, (short)0, g.nx * g.ny * g.nz * 4, 0x00020000)};
 }
 
-// trilinear_interpolate, src/Grid.h:94-108
+// trilinear_interpolate, src/Grid.h:94-108 (the lower cell is at most nx - 2)
 template <class S, class L>
 __device__ __forceinline__ float trilinear_g(const Gv& g, const L& ldg, const S& sc, f3 p) {
     const float gX = fmaxf(fminf(sc(p.x) - g.ox, (float)g.nx - 1.001f), 0.0f);
@@ -104,10 +115,11 @@ __device__ __forceinline__ float trilinear_g(const Gv& g, const L& ldg, const S&
     const float tx = gX - (float)i, ty = gY - (float)j, tz = gZ - (float)k;
     const int sy = g.nx, sz = g.nx * g.ny;
     const int b = i + j * sy + k * sz;
-    const float c00 = ldg(b) * (1.0f - tx) + ldg(b + 1) * tx;
-    const float c10 = ldg(b + sy) * (1.0f - tx) + ldg(b + sy + 1) * tx;
-    const float c01 = ldg(b + sz) * (1.0f - tx) + ldg(b + sz + 1) * tx;
-    const float c11 = ldg(b + sy + sz) * (1.0f - tx) + ldg(b + sy + sz + 1) * tx;
+    const f32x2 q00 = ldg.two(b), q10 = ldg.two(b + sy), q01 = ldg.two(b + sz), q11 = ldg.two(b + sy + sz);
+    const float c00 = q00[0] * (1.0f - tx) + q00[1] * tx;
+    const float c10 = q10[0] * (1.0f - tx) + q10[1] * tx;
+    const float c01 = q01[0] * (1.0f - tx) + q01[1] * tx;
+    const float c11 = q11[0] * (1.0f - tx) + q11[1] * tx;
     return (1.0f - tz) * ((1.0f - ty) * c00 + ty * c10) + tz * ((1.0f - ty) * c01 + ty * c11);
 }
 template <class S>
@@ -143,7 +155,10 @@ __device__ __forceinline__ float cw_apply(const CW& c, float q0, float q1, float
 }
 
 // tricubic_interpolate, src/Grid.h:165-222: x cerps, then y, then z; with
-// clamp, every 1-D stage is clamped at 0 (cerpc).
+// clamp, every 1-D stage is clamped at 0 (cerpc). The four nodes of a row
+// are one load (a row has at least four elements); where the first or last
+// repeats the grid's edge, the load moves inside the row and the nodes are
+// picked from it.
 template <bool CLAMP, class S, class L>
 __device__ __forceinline__ float tricubic_g(const Gv& g, const L& ldg, const S& sc, f3 p) {
     const float gX = fmaxf(fminf(sc(p.x) - g.ox, (float)g.nx - 1.001f), 0.0f);
@@ -151,25 +166,34 @@ __device__ __forceinline__ float tricubic_g(const Gv& g, const L& ldg, const S& 
     const float gZ = fmaxf(fminf(sc(p.z) - g.oz, (float)g.nz - 1.001f), 0.0f);
     const int i1 = (int)gX, j1 = (int)gY, k1 = (int)gZ;
     const int sy = g.nx, sz = g.nx * g.ny;
-    const int ix[4] = {max(i1 - 1, 0), i1, i1 + 1, min(i1 + 2, g.nx - 1)};
+    const int ix = min(max(i1 - 1, 0), g.nx - 4);
+    const bool low = i1 < 1, high = i1 > g.nx - 3;
     const int jy[4] = {max(j1 - 1, 0) * sy, j1 * sy, (j1 + 1) * sy, min(j1 + 2, g.ny - 1) * sy};
     const int kz[4] = {max(k1 - 1, 0) * sz, k1 * sz, (k1 + 1) * sz, min(k1 + 2, g.nz - 1) * sz};
     const CW cx = cw(gX - (float)i1), cy = cw(gY - (float)j1), cz = cw(gZ - (float)k1);
-    float rz[4];
+    auto sample = [&](auto edge) {
+        float rz[4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        float ry[4];
+        for (int c = 0; c < 4; ++c) {
+            float ry[4];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int row = jy[b] + kz[c];
-            float v = cw_apply(cx, ldg(row + ix[0]), ldg(row + ix[1]), ldg(row + ix[2]), ldg(row + ix[3]));
-            ry[b] = CLAMP ? fmaxf(v, 0.0f) : v;
+            for (int b = 0; b < 4; ++b) {
+                f32x4 q = ldg.four(jy[b] + kz[c] + ix);
+                if (edge())
+                    q = f32x4{high ? q[1] : q[0], low ? q[0] : (high ? q[2] : q[1]), low ? q[1] : (high ? q[3] : q[2]),
+                              low ? q[2] : q[3]};
+                float v = cw_apply(cx, q[0], q[1], q[2], q[3]);
+                ry[b] = CLAMP ? fmaxf(v, 0.0f) : v;
+            }
+            float v = cw_apply(cy, ry[0], ry[1], ry[2], ry[3]);
+            rz[c] = CLAMP ? fmaxf(v, 0.0f) : v;
         }
-        float v = cw_apply(cy, ry[0], ry[1], ry[2], ry[3]);
-        rz[c] = CLAMP ? fmaxf(v, 0.0f) : v;
-    }
-    float v = cw_apply(cz, rz[0], rz[1], rz[2], rz[3]);
-    return CLAMP ? fmaxf(v, 0.0f) : v;
+        float v = cw_apply(cz, rz[0], rz[1], rz[2], rz[3]);
+        return CLAMP ? fmaxf(v, 0.0f) : v;
+    };
+    // one way for the whole wave: most have no lane at an edge
+    if (__any(low || high)) return sample([] { return true; });
+    return sample([] { return false; });
 }
 template <bool CLAMP, class S>
 __device__ __forceinline__ float tricubic_s(const Gv& g, const S& sc, f3 p) {

@@ -7,6 +7,13 @@
 // buffer; the host swaps front/back pointers afterwards (no device kernel).
 // Positions are scaled to grid units by p / dx, or by p * 2^k when dx =
 // 2^-k (the same bits, without 30 IEEE divisions per cell).
+//
+// Bound by the L1's accesses (one per clock and CU): 72 velocity and 64 field
+// elements per cell. With two and four of a row per load, a component of 256^3
+// takes 510 us and temperature with smoke 790; one element per load, bound by
+// the rate of load instructions, took 680 and 1110. Giving each XCD one run of
+// neighbouring rows (560 and 940) or larger workgroups lost: neighbouring
+// planes at the same time on all XCDs is better for the shared cache.
 #include "solver.h"
 
 namespace blz {
