@@ -11,11 +11,15 @@
 // a stable radix sort by cell key (k_sort.hip) keeps ascending particle
 // order inside each cell; one thread per cell then sums its run
 // sequentially from +0 and overwrites the front value when |sum| > 1e-5.
-// The entry buffers are sized from a host-side upper bound of the
-// footprints (p2g_entry_bound), so no count is read back mid-pipeline. Cells that receive nothing keep their front value, exactly
-// as the reference's copy-where-nonzero does. The reference's back buffers
-// after addSource are dead (every later reader overwrites them first), so
-// no full-grid clear or copy pass is needed.
+// The entries of a particle set are counted once, when it arrives
+// (p2g_measure), and the buffers and launches of its splats sized by that
+// count: one read-back per upload. (Sized by an upper bound of the footprints,
+// the sort of a million particles of 0.6 cells ran 0.6 ms over 40 entries per
+// particle where few are, and adding up the bound on the host took 1.2 ms.)
+// Cells that receive nothing keep their front value, exactly as the
+// reference's copy-where-nonzero does. The reference's back buffers after
+// addSource are dead (every later reader overwrites them first), so no
+// full-grid clear or copy pass is needed.
 #include <cmath>
 
 #include "solver.h"
@@ -26,6 +30,12 @@ namespace {
 
 constexpr unsigned BS = 256;
 constexpr int NCH = 5; // T, U, V, W, smoke density
+
+// what the host reads once the stream is idle
+struct P2GHost {
+    unsigned long long bound;
+    unsigned total, overflow;
+};
 
 struct PGrid {
     int nx, ny, nz;
@@ -95,7 +105,30 @@ __device__ __forceinline__ void footprint(const float* r, const PGrid& g, const 
             }
 }
 
+// Upper bound of a particle set's (cell, value) entries, added to *bound: a
+// particle that passes the pscale > dx/2 gate (:83) covers at most
+// floor(pscale/dx + 0.01) + 2 cells per axis of a channel's grid (the
+// footprint box of sphereToGrid, src/Grid.h:315-324, spans pscale/dx cells
+// up to float rounding, plus the truncation of both ends), in each of the
+// nch channels. Sets above P2G_MAX entries are refused before any footprint
+// is walked.
+constexpr unsigned long long P2G_MAX = 0x7fffffffull;
+constexpr int BOUND_BLOCKS = 512;
+__global__ void __launch_bounds__(BS) k_p2g_bound(const float* __restrict__ part, int n, float dx, int nch,
+                                                  unsigned long long* __restrict__ bound) {
+    unsigned long long b = 0;
+    for (long long q = (long long)blockIdx.x * BS + threadIdx.x; q < n; q += (long long)gridDim.x * BS) {
+        const float ps = part[(size_t)q * 8 + 6];
+        if (!(ps > dx / 2.0f)) continue;
+        const double w = floor((double)ps / (double)dx + 0.01) + 2.0;
+        b += (unsigned long long)fmin(w * w * w, 4294967296.0) * (unsigned long long)nch;
+    }
+    for (int o = 32; o >= 1; o >>= 1) b += __shfl_xor(b, o, 64);
+    if ((threadIdx.x & 63) == 0 && b) atomicAdd(bound, b); // integers: any order gives the same sum
+}
+
 __global__ void __launch_bounds__(BS) k_p2g_count(const float* __restrict__ part, int n, P2G P,
+                                                  const unsigned long long* __restrict__ bound,
                                                   unsigned* __restrict__ counts) {
     const int t = blockIdx.x * BS + threadIdx.x;
     if (t >= n * P.nch) return;
@@ -103,6 +136,10 @@ __global__ void __launch_bounds__(BS) k_p2g_count(const float* __restrict__ part
     const float* r = part + (size_t)q * 8;
     float val;
     unsigned c = 0;
+    if (bound && *bound > P2G_MAX) {
+        counts[t] = 0u;
+        return;
+    }
     if (channel_value(r, ch, P, &val)) footprint(r, P.g[ch], P, val, [&](int, float) { ++c; });
     counts[t] = c;
 }
@@ -119,7 +156,7 @@ __global__ void __launch_bounds__(BS) k_p2g_emit(const float* __restrict__ part,
     unsigned o = offs[t];
     const unsigned base = P.g[ch].base;
     footprint(r, P.g[ch], P, val, [&](int cell, float v) {
-        if (o < cap) { // the host bound makes this always true (k_p2g_total flags the contrary)
+        if (o < cap) { // the count of the set makes this always true (k_p2g_total flags the contrary)
             keys[o] = base + (unsigned)cell;
             vals[o] = v;
         }
@@ -128,13 +165,19 @@ __global__ void __launch_bounds__(BS) k_p2g_emit(const float* __restrict__ part,
 }
 
 // the entry count the sort and the reduction use: the total of the scan,
-// clamped to the buffers (a total above them, which the host bound rules
-// out, is flagged and the splat reported as failed)
+// clamped to the buffers (a total above them, which the count of the set
+// rules out, is flagged and the splat reported as failed)
 __global__ void k_p2g_total(const unsigned* __restrict__ total, unsigned cap, unsigned* __restrict__ n_out,
-                            unsigned* __restrict__ overflow) {
+                            P2GHost* __restrict__ host) {
     const unsigned t = *total;
     *n_out = t < cap ? t : cap;
-    *overflow = t > cap ? 1u : 0u;
+    host->overflow = t > cap ? 1u : 0u;
+}
+__global__ void k_p2g_clear(unsigned long long* bound) { *bound = 0ull; }
+__global__ void k_p2g_measured(const unsigned* __restrict__ total, const unsigned long long* __restrict__ bound,
+                               P2GHost* __restrict__ host) {
+    host->total = *total;
+    host->bound = *bound;
 }
 
 // one thread per run of equal keys: sequential sum in particle order
@@ -171,6 +214,7 @@ int ensure(Solver& s, void** p, size_t* cap, size_t need) {
 }
 
 struct Scratch {
+    P2GHost* host = nullptr; // pinned
     void* counts = nullptr; size_t counts_cap = 0;   // counts, offsets, scan scratch, totals
     void* entries = nullptr; size_t entries_cap = 0; // keys, values and their sorted copies
     void* sort = nullptr; size_t sort_cap = 0;       // radix sort scratch
@@ -194,6 +238,7 @@ static Scratch& scratch_of(Solver& s) {
 void free_p2g_scratch(Solver& s) {
     if (!s.p2g_buf) return;
     Scratch* sc = (Scratch*)s.p2g_buf;
+    if (sc->host) (void)hipHostFree(sc->host);
     if (sc->counts) (void)hipFree(sc->counts);
     if (sc->entries) (void)hipFree(sc->entries);
     if (sc->sort) (void)hipFree(sc->sort);
@@ -201,27 +246,7 @@ void free_p2g_scratch(Solver& s) {
     s.p2g_buf = nullptr;
 }
 
-// Upper bound of the (cell, value) entries of a particle set, on the host:
-// a particle that passes the pscale > dx/2 gate (:83) covers at most
-// floor(pscale/dx + 0.01) + 2 cells per axis of a channel's grid (the
-// footprint box of sphereToGrid, src/Grid.h:315-324, spans pscale/dx cells
-// up to float rounding, plus the truncation of both ends), in each of the
-// nch channels.
-size_t p2g_entry_bound(const float* part8, int n, float dx, int nch) {
-    size_t b = 0;
-    for (int q = 0; q < n; ++q) {
-        const float ps = part8[(size_t)q * 8 + 6];
-        if (!(ps > dx / 2.0f)) continue;
-        const double w = std::floor((double)ps / (double)dx + 0.01) + 2.0;
-        b += (size_t)(w * w * w) * (size_t)nch;
-    }
-    return b;
-}
-
-int launch_p2g(Solver& s) {
-    const int n = s.npart;
-    if (n <= 0) return BLZ_OK;
-    Scratch& sc = scratch_of(s);
+static P2G grids_of(const Solver& s, unsigned* key_end) {
     P2G P{};
     P.nch = s.smoke ? 5 : 4;
     P.dx = s.dx;
@@ -236,48 +261,99 @@ int launch_p2g(Solver& s) {
         P.g[g] = PGrid{F.nx, F.ny, F.nz, F.ox, F.oy, F.oz, F.flip ? 1 : 0, base, F.front()};
         base += (unsigned)F.count();
     }
-    const unsigned key_end = base;
-    int end_bit = 1;
-    while (end_bit < 32 && (1ull << end_bit) < (unsigned long long)key_end) ++end_bit;
-    const size_t bound = s.p2g_bound;
-    if (bound == 0) return BLZ_OK; // no particle passes the pscale gate
-    if (bound > 0x7fffffffu) {
+    *key_end = base;
+    return P;
+}
+
+// counts (m), offsets (m + 1, the total last), scan scratch, the clamped
+// total, the bound
+struct Counts {
+    size_t m;
+    unsigned *counts, *offs, *scan_tmp, *n_eff;
+    unsigned long long* bound;
+};
+static int counts_of(Solver& s, int nch, Scratch& sc, Counts* c) {
+    c->m = (size_t)s.npart * nch;
+    const size_t scw = scan_scratch_words(c->m), words = (2 * c->m + 1 + scw + 1 + 1) / 2 * 2;
+    if (int e = ensure(s, &sc.counts, &sc.counts_cap, (words + 2) * sizeof(unsigned))) return e;
+    if (!sc.host) BLZ_HIP(hipHostMalloc((void**)&sc.host, sizeof(P2GHost), hipHostMallocDefault));
+    c->counts = (unsigned*)sc.counts;
+    c->offs = c->counts + c->m;
+    c->scan_tmp = c->offs + c->m + 1;
+    c->n_eff = c->scan_tmp + scw;
+    c->bound = (unsigned long long*)(c->counts + words);
+    return BLZ_OK;
+}
+
+// The bound and the entries of the particle set in s.part (s.p2g_bound,
+// s.p2g_entries), with the counts and offsets left for the splat that
+// follows; waits for the solver's stream
+int p2g_measure(Solver& s) {
+    s.p2g_bound = 0;
+    s.p2g_entries = 0;
+    const int n = s.npart;
+    if (n <= 0) return BLZ_OK;
+    unsigned key_end = 0;
+    const P2G P = grids_of(s, &key_end);
+    Scratch& sc = scratch_of(s);
+    Counts c;
+    if (int e = counts_of(s, P.nch, sc, &c)) return e;
+    hipLaunchKernelGGL(k_p2g_clear, dim3(1), dim3(1), 0, s.stream, c.bound);
+    hipLaunchKernelGGL(k_p2g_bound, dim3(std::min<unsigned>(BOUND_BLOCKS, blocks_for(n, BS))), dim3(BS), 0, s.stream,
+                       s.part, n, s.dx, P.nch, c.bound);
+    hipLaunchKernelGGL(k_p2g_count, dim3(blocks_for(c.m, BS)), dim3(BS), 0, s.stream, s.part, n, P, c.bound, c.counts);
+    BLZ_HIP(hipGetLastError());
+    if (int e = scan_exclusive(s.stream, c.counts, c.offs, nullptr, c.m, c.scan_tmp)) return e;
+    hipLaunchKernelGGL(k_p2g_measured, dim3(1), dim3(1), 0, s.stream, c.offs + c.m, c.bound, sc.host);
+    BLZ_HIP(hipGetLastError());
+    BLZ_HIP(hipStreamSynchronize(s.stream));
+    s.p2g_bound = (size_t)sc.host->bound;
+    s.p2g_entries = (size_t)sc.host->total;
+    return BLZ_OK;
+}
+
+// counted: p2g_measure has just left the counts and offsets
+int launch_p2g(Solver& s, bool counted) {
+    const int n = s.npart;
+    if (n <= 0) return BLZ_OK;
+    if (s.p2g_bound > P2G_MAX) {
         set_error("particle-to-grid footprint bound exceeds 2^31 entries");
         return BLZ_E_INVALID;
     }
-
-    // counts (m), offsets (m + 1, the total last), scan scratch, the clamped
-    // total and the overflow flag
-    const size_t m = (size_t)n * P.nch;
-    const size_t scw = scan_scratch_words(m);
-    if (int e = ensure(s, &sc.counts, &sc.counts_cap, (2 * m + 1 + scw + 2) * sizeof(unsigned))) return e;
-    unsigned* counts = (unsigned*)sc.counts;
-    unsigned* offs = counts + m;
-    unsigned* scan_tmp = offs + m + 1;
-    unsigned* n_eff = scan_tmp + scw;
-    unsigned* overflow = n_eff + 1;
-    if (int e = ensure(s, &sc.entries, &sc.entries_cap, bound * 16)) return e;
-    if (int e = ensure(s, &sc.sort, &sc.sort_cap, radix_scratch_words(bound) * sizeof(unsigned))) return e;
+    const size_t cap = s.p2g_entries;
+    if (cap == 0) return BLZ_OK; // no particle reaches a cell
+    unsigned key_end = 0;
+    const P2G P = grids_of(s, &key_end);
+    int end_bit = 1;
+    while (end_bit < 32 && (1ull << end_bit) < (unsigned long long)key_end) ++end_bit;
+    Scratch& sc = scratch_of(s);
+    Counts c;
+    if (int e = counts_of(s, P.nch, sc, &c)) return e;
+    if (int e = ensure(s, &sc.entries, &sc.entries_cap, cap * 16)) return e;
+    if (int e = ensure(s, &sc.sort, &sc.sort_cap, radix_scratch_words(cap) * sizeof(unsigned))) return e;
     unsigned* keys_in = (unsigned*)sc.entries;
-    unsigned* keys_out = keys_in + bound;
-    float* vals_in = (float*)(keys_out + bound);
-    float* vals_out = vals_in + bound;
+    unsigned* keys_out = keys_in + cap;
+    float* vals_in = (float*)(keys_out + cap);
+    float* vals_out = vals_in + cap;
 
-    hipLaunchKernelGGL(k_p2g_count, dim3(blocks_for(m, BS)), dim3(BS), 0, s.stream, s.part, n, P, counts);
-    BLZ_HIP(hipGetLastError());
-    if (int e = scan_exclusive(s.stream, counts, offs, nullptr, m, scan_tmp)) return e;
-    hipLaunchKernelGGL(k_p2g_total, dim3(1), dim3(1), 0, s.stream, offs + m, (unsigned)bound, n_eff, overflow);
-    hipLaunchKernelGGL(k_p2g_emit, dim3(blocks_for(m, BS)), dim3(BS), 0, s.stream, s.part, n, P, offs,
-                       (unsigned)bound, keys_in, vals_in);
+    if (!counted) {
+        hipLaunchKernelGGL(k_p2g_count, dim3(blocks_for(c.m, BS)), dim3(BS), 0, s.stream, s.part, n, P,
+                           (const unsigned long long*)nullptr, c.counts);
+        BLZ_HIP(hipGetLastError());
+        if (int e = scan_exclusive(s.stream, c.counts, c.offs, nullptr, c.m, c.scan_tmp)) return e;
+    }
+    hipLaunchKernelGGL(k_p2g_total, dim3(1), dim3(1), 0, s.stream, c.offs + c.m, (unsigned)cap, c.n_eff, sc.host);
+    hipLaunchKernelGGL(k_p2g_emit, dim3(blocks_for(c.m, BS)), dim3(BS), 0, s.stream, s.part, n, P, c.offs,
+                       (unsigned)cap, keys_in, vals_in);
     BLZ_HIP(hipGetLastError());
     bool alt = false;
-    if (int e = radix_sort_pairs(s.stream, keys_in, vals_in, keys_out, vals_out, n_eff, bound, end_bit,
+    if (int e = radix_sort_pairs(s.stream, keys_in, vals_in, keys_out, vals_out, c.n_eff, cap, end_bit,
                                  (unsigned*)sc.sort, &alt))
         return e;
-    hipLaunchKernelGGL(k_p2g_reduce, dim3(blocks_for(bound, BS)), dim3(BS), 0, s.stream, alt ? keys_out : keys_in,
-                       alt ? vals_out : vals_in, n_eff, P);
+    hipLaunchKernelGGL(k_p2g_reduce, dim3(blocks_for(cap, BS)), dim3(BS), 0, s.stream, alt ? keys_out : keys_in,
+                       alt ? vals_out : vals_in, c.n_eff, P);
     BLZ_HIP(hipGetLastError());
-    s.p2g_overflow = overflow;
+    s.p2g_overflow = &sc.host->overflow;
     return BLZ_OK;
 }
 

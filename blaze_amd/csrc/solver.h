@@ -208,9 +208,11 @@ struct Solver {
     // particle-to-grid scratch (grow-only)
     void* p2g_buf = nullptr;
     size_t p2g_bytes = 0;
-    size_t p2g_bound = 0;              // upper bound of the splat's entries (host, from the particle set)
-    size_t stage_bound[2] = {0, 0};    // the same for each staged slot
-    const unsigned* p2g_overflow = nullptr; // device flag of the last splat: its entries exceeded the bound
+    // of the particle set (p2g_measure): an upper bound of its splat's entries
+    // and their number; p2g_new: a set that has not been measured
+    size_t p2g_bound = 0, p2g_entries = 0;
+    bool p2g_new = false;
+    const unsigned* p2g_overflow = nullptr; // pinned flag of the last splat: its entries exceeded their number
     // stats / timing: spans of device work bracketed by pooled events,
     // resolved after the stream has been synchronised (no extra waits)
     blz_stats st{};
@@ -408,8 +410,8 @@ void ctl_reset_jobs(Solver& s, SolveCtl* c, std::vector<CtlJob>& jobs, bool adap
 int launch_buoyancy_multi(hipStream_t st, bool mul, const BuoyJob* tab, int n, int blocks);
 int launch_divergence_multi(hipStream_t st, const DivJob* tab, int n, int blocks);
 int launch_ctl_reset_multi(hipStream_t st, const CtlJob* tab, int n);
-int launch_p2g(Solver& s);
-size_t p2g_entry_bound(const float* part8, int n, float dx, int nch);
+int p2g_measure(Solver& s);
+int launch_p2g(Solver& s, bool counted);
 int launch_max_abs_velocity(Solver& s, double* dev_out);
 int launch_clear_doubles(Solver& s, double* dev, int n);
 int launch_p_to_natural(Solver& s, float* out, const RB& src);
