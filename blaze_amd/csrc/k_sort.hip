@@ -104,6 +104,51 @@ __global__ void __launch_bounds__(SB) k_scan_tiles(const unsigned* __restrict__ 
     }
 }
 
+// The whole scan in one workgroup, ONE_THREADS * SCAN_ITEMS elements per round.
+// Up to ONE_MAX elements (two rounds: 3.5 us for one, 7.4 for both) it beats
+// the three launches above, which a source pays four times per splat: 9 us for
+// some 10^4 elements, 14 at 3 * 10^4. Four rounds take 25 to 34 us.
+constexpr int ONE_THREADS = 1024;
+constexpr size_t ONE_MAX = 2 * (size_t)ONE_THREADS * SCAN_ITEMS;
+__global__ void __launch_bounds__(ONE_THREADS) k_scan_one(const unsigned* __restrict__ in,
+                                                          const unsigned* __restrict__ n_dev, size_t n_host,
+                                                          unsigned* __restrict__ out) {
+    __shared__ unsigned sm[ONE_THREADS / 64];
+    const size_t n = n_dev ? (size_t)*n_dev : n_host;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    unsigned carry = 0;
+    for (size_t b0 = 0; b0 <= n; b0 += (size_t)ONE_THREADS * SCAN_ITEMS) {
+        const size_t base = b0 + (size_t)threadIdx.x * SCAN_ITEMS;
+        unsigned v[SCAN_ITEMS], s = 0;
+#pragma unroll
+        for (int i = 0; i < SCAN_ITEMS; ++i) {
+            v[i] = base + i < n ? in[base + i] : 0u;
+            s += v[i];
+        }
+        unsigned x = s;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+        if (lane == 63) sm[w] = x;
+        __syncthreads();
+        unsigned run = carry + x - s;
+#pragma unroll
+        for (int q = 0; q < ONE_THREADS / 64; ++q) {
+            if (q < w) run += sm[q];
+            carry += sm[q];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < SCAN_ITEMS; ++i) {
+            if (base + i < n) out[base + i] = run;
+            if (base + i == n) out[n] = run; // the total
+            run += v[i];
+        }
+    }
+}
+
 // the sort's digit histogram of each tile: hist[d * ntiles + tile]
 __global__ void __launch_bounds__(SB) k_radix_hist(const unsigned* __restrict__ keys, const unsigned* __restrict__ n_dev,
                                                    int shift, unsigned* __restrict__ hist, int ntiles) {
@@ -121,33 +166,44 @@ __global__ void __launch_bounds__(SB) k_radix_hist(const unsigned* __restrict__ 
     hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
-// Stable scatter of a tile by one digit. The tile's elements are taken in
-// rounds i = 0..SORT_ITEMS-1, element base + i * SB + thread, which is the
-// input order (round, wave, lane). In a round each lane finds the lanes of
-// its wave holding the same digit (eight ballots, one per digit bit); its
-// destination is the digit's global offset (scanned histogram) + the
-// elements of that digit in earlier rounds + in earlier waves of this round
-// + on lower lanes of its wave.
+// Stable scatter of a tile by one digit. Wave w takes the w-th run of
+// SORT_ITEMS * 64 elements, 64 per round, so the input order is (wave, round,
+// lane). In a round each lane finds the lanes of its wave holding the same
+// digit (eight ballots, one per digit bit); its place among the wave's
+// elements of that digit is the digit's count in earlier rounds, kept per wave
+// in LDS, + the holders on lower lanes. Its destination is the digit's global
+// offset (scanned histogram) + the elements of that digit in earlier waves +
+// that place. The rounds need no barrier between them: one for each tile-wide
+// round made the launch 7.2 us for 10^4 pairs, now
+// 4.6.
 __global__ void __launch_bounds__(SB) k_radix_scatter(const unsigned* __restrict__ keys_in,
                                                       const float* __restrict__ vals_in,
                                                       const unsigned* __restrict__ n_dev, int shift,
                                                       const unsigned* __restrict__ hist_scan, int ntiles,
                                                       unsigned* __restrict__ keys_out, float* __restrict__ vals_out) {
-    __shared__ unsigned run[RADIX];        // offset of each digit for the next element
-    __shared__ unsigned wc[WAVES][RADIX];  // per round: elements of each digit per wave
+    __shared__ unsigned wc[WAVES][RADIX]; // elements of each digit per wave, then their first destination
     const size_t n = *n_dev;
     const size_t base = (size_t)blockIdx.x * SORT_TILE;
     if (base >= n) return; // whole block: uniform
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    run[threadIdx.x] = hist_scan[(size_t)threadIdx.x * ntiles + blockIdx.x];
+    const unsigned first = hist_scan[(size_t)threadIdx.x * ntiles + blockIdx.x];
     const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
+    const size_t e0 = base + (size_t)w * (SORT_ITEMS * 64) + lane;
+    unsigned key[SORT_ITEMS], place[SORT_ITEMS];
+    float val[SORT_ITEMS];
+#pragma unroll
     for (int i = 0; i < SORT_ITEMS; ++i) {
-        for (int q = 0; q < WAVES; ++q) wc[q][threadIdx.x] = 0u;
-        __syncthreads();
-        const size_t e = base + (size_t)i * SB + threadIdx.x;
-        const bool ok = e < n;
-        const unsigned key = ok ? keys_in[e] : 0u;
-        const unsigned d = (key >> shift) & (RADIX - 1);
+        const size_t e = e0 + (size_t)i * 64;
+        key[i] = e < n ? keys_in[e] : 0u;
+        val[i] = e < n ? vals_in[e] : 0.0f;
+    }
+#pragma unroll
+    for (int q = 0; q < WAVES; ++q) wc[q][threadIdx.x] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < SORT_ITEMS; ++i) {
+        const bool ok = e0 + (size_t)i * 64 < n;
+        const unsigned d = (key[i] >> shift) & (RADIX - 1);
         unsigned long long peers = __ballot(ok);
 #pragma unroll
         for (int b = 0; b < RADIX_BITS; ++b) {
@@ -155,21 +211,30 @@ __global__ void __launch_bounds__(SB) k_radix_scatter(const unsigned* __restrict
             peers &= ((d >> b) & 1u) ? m : ~m;
         }
         const unsigned rank = (unsigned)__popcll(peers & below);
-        if (ok && rank == 0) wc[w][d] = (unsigned)__popcll(peers);
-        __syncthreads();
-        if (ok) {
-            unsigned off = run[d] + rank;
-            for (int q = 0; q < w; ++q) off += wc[q][d];
-            if (off < n) {
-                keys_out[off] = key;
-                vals_out[off] = vals_in[e];
-            }
+        const unsigned before = wc[w][d];
+        place[i] = before + rank;
+        // the row is this wave's own: its reads above come before the write
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (ok && rank == 0) wc[w][d] = before + (unsigned)__popcll(peers);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    __syncthreads();
+    unsigned off = first;
+#pragma unroll
+    for (int q = 0; q < WAVES; ++q) {
+        const unsigned c = wc[q][threadIdx.x];
+        wc[q][threadIdx.x] = off;
+        off += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < SORT_ITEMS; ++i) {
+        if (e0 + (size_t)i * 64 >= n) continue;
+        const unsigned o = wc[w][(key[i] >> shift) & (RADIX - 1)] + place[i];
+        if (o < n) {
+            keys_out[o] = key[i];
+            vals_out[o] = val[i];
         }
-        __syncthreads();
-        unsigned add = 0;
-        for (int q = 0; q < WAVES; ++q) add += wc[q][threadIdx.x];
-        run[threadIdx.x] += add;
-        __syncthreads();
     }
 }
 
@@ -184,6 +249,11 @@ size_t scan_scratch_words(size_t n_max) { return tiles_of(n_max + 1, SCAN_TILE) 
 int scan_exclusive(hipStream_t st, const unsigned* in, unsigned* out, const unsigned* n_dev, size_t n_max,
                    unsigned* scratch) {
     const unsigned nt = tiles_of(n_max + 1, SCAN_TILE);
+    if (n_max < ONE_MAX) {
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(ONE_THREADS), 0, st, in, n_dev, n_max, out);
+        BLZ_HIP(hipGetLastError());
+        return BLZ_OK;
+    }
     hipLaunchKernelGGL(k_scan_sums, dim3(nt), dim3(SB), 0, st, in, n_dev, n_max, scratch);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(SB), 0, st, scratch, (int)nt);
     hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(SB), 0, st, in, n_dev, n_max, scratch, out);
