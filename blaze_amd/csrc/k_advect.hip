@@ -54,12 +54,6 @@ __device__ __forceinline__ void advect_cell(const Gv& U, const Gv& V, const Gv& 
     as_global(out)[t] = tricubic_s<CLAMP>(G, sc, pos);
 }
 
-template <bool CLAMP, class S>
-__global__ void __launch_bounds__(BS) k_advect(Gv U, Gv V, Gv W, Gv G, float* __restrict__ out, S sc, float dx,
-                                               float a, float b, float c1, float c2, float c3, float dt) {
-    advect_cell<CLAMP>(U, V, W, G, out, sc, dx, a, b, c1, c2, c3, dt, (int)(blockIdx.x * BS + threadIdx.x));
-}
-
 // temperature and smoke density share the cell-centred grid, hence the
 // back-trace: one trace, two clamped tricubic samples (the same values as
 // two separate launches)
@@ -76,11 +70,32 @@ __device__ __forceinline__ void advect_pair_cell(const Gv& U, const Gv& V, const
     as_global(out2)[t] = tricubic_s<true>(G2, sc, pos);
 }
 
-template <class S>
-__global__ void __launch_bounds__(BS) k_advect_pair(Gv U, Gv V, Gv W, Gv G1, Gv G2, float* __restrict__ out1,
-                                                    float* __restrict__ out2, S sc, float dx, float a, float b,
-                                                    float c1, float c2, float c3, float dt) {
-    advect_pair_cell(U, V, W, G1, G2, out1, out2, sc, dx, a, b, c1, c2, c3, dt, (int)(blockIdx.x * BS + threadIdx.x));
+// Every advected field of a grid in one launch, the longest first (a launch
+// per field left most CUs idle at 32^3: 33 us for four, 11 together; at 256^3
+// with smoke 2310 and 2100)
+struct AdvAll {
+    Gv U, V, W, T, D;
+    float *oT, *oD, *oF[3];
+    int first[3]; // first block of each velocity component
+    float dx, a, b, dt;
+};
+template <bool PAIR, class S>
+__global__ void __launch_bounds__(BS, 6) k_advect(AdvAll e, S sc) {
+    const int b = (int)blockIdx.x;
+    if (b < e.first[0]) {
+        const int t = b * (int)BS + (int)threadIdx.x;
+        if (PAIR)
+            advect_pair_cell(e.U, e.V, e.W, e.T, e.D, e.oT, e.oD, sc, e.dx, e.a, e.b, RK_C1, RK_C2, RK_C3, e.dt, t);
+        else
+            advect_cell<true>(e.U, e.V, e.W, e.T, e.oT, sc, e.dx, e.a, e.b, RK_C1, RK_C2, RK_C3, e.dt, t);
+        return;
+    }
+    const int c = b < e.first[1] ? 0 : (b < e.first[2] ? 1 : 2);
+    const Gv& G = c == 0 ? e.U : (c == 1 ? e.V : e.W);
+    const int first = c == 0 ? e.first[0] : (c == 1 ? e.first[1] : e.first[2]);
+    float* out = c == 0 ? e.oF[0] : (c == 1 ? e.oF[1] : e.oF[2]);
+    advect_cell<false>(e.U, e.V, e.W, G, out, sc, e.dx, e.a, e.b, RK_C1, RK_C2, RK_C3, e.dt,
+                       (b - first) * (int)BS + (int)threadIdx.x);
 }
 
 // the job of block b in a table of first blocks (ascending)
@@ -109,30 +124,29 @@ __global__ void __launch_bounds__(BS) k_advect_multi(const AdvJob* __restrict__ 
 
 template <class S>
 int advect_all(Solver& s, const S& sc, float dt) {
-    const Gv U = s.f[F_U].view(), V = s.f[F_V].view(), W = s.f[F_W].view();
-    const float a = 0.5f * dt, b = 0.75f * dt;
-    const float c1 = RK_C1, c2 = RK_C2, c3 = RK_C3;
-    for (int g = F_T; g < F_N; ++g) {
-        Field& G = s.f[g];
-        const size_t n = G.count();
-        if (g == F_S && !s.smoke) continue;
-        const Gv tv = s.f[F_T].view(), dv = s.f[F_S].view();
-        const bool pair = s.smoke && tv.nx == dv.nx && tv.ny == dv.ny && tv.nz == dv.nz && tv.ox == dv.ox &&
-                          tv.oy == dv.oy && tv.oz == dv.oz;
-        if (g == F_S && pair) continue; // with T
-        if (g == F_T && pair) {
-            Field& D = s.f[F_S];
-            hipLaunchKernelGGL(k_advect_pair<S>, dim3(blocks_for(n, BS)), dim3(BS), 0, s.stream, U, V, W, G.view(),
-                               D.view(), G.back(), D.back(), sc, s.dx, a, b, c1, c2, c3, dt);
-        } else if (g == F_T || g == F_S) {
-            hipLaunchKernelGGL((k_advect<true, S>), dim3(blocks_for(n, BS)), dim3(BS), 0, s.stream, U, V, W, G.view(),
-                               G.back(), sc, s.dx, a, b, c1, c2, c3, dt);
-        } else {
-            hipLaunchKernelGGL((k_advect<false, S>), dim3(blocks_for(n, BS)), dim3(BS), 0, s.stream, U, V, W,
-                               G.view(), G.back(), sc, s.dx, a, b, c1, c2, c3, dt);
-        }
-        BLZ_HIP(hipGetLastError());
+    AdvAll e{};
+    e.U = s.f[F_U].view();
+    e.V = s.f[F_V].view();
+    e.W = s.f[F_W].view();
+    e.T = s.f[F_T].view();
+    e.oT = s.f[F_T].back();
+    if (s.smoke) {
+        e.D = s.f[F_S].view();
+        e.oD = s.f[F_S].back();
     }
+    unsigned blocks = blocks_for(s.f[F_T].count(), BS);
+    for (int c = 0; c < 3; ++c) {
+        e.oF[c] = s.f[F_U + c].back();
+        e.first[c] = (int)blocks;
+        blocks += blocks_for(s.f[F_U + c].count(), BS);
+    }
+    e.dx = s.dx;
+    e.a = 0.5f * dt;
+    e.b = 0.75f * dt;
+    e.dt = dt;
+    if (s.smoke) hipLaunchKernelGGL((k_advect<true, S>), dim3(blocks), dim3(BS), 0, s.stream, e, sc);
+    else hipLaunchKernelGGL((k_advect<false, S>), dim3(blocks), dim3(BS), 0, s.stream, e, sc);
+    BLZ_HIP(hipGetLastError());
     return BLZ_OK;
 }
 

@@ -144,10 +144,9 @@ __global__ void __launch_bounds__(BS) k_vort_force(float dx, float* __restrict__
 // RANGE2: only cells 2..N-3 on every axis carry increments (vorticity);
 // otherwise every cell does (curl noise).
 template <int AXIS, bool RANGE2>
-__global__ void __launch_bounds__(BS) k_face_gather(float* __restrict__ face, const float* __restrict__ inc,
-                                                    int nW, int nH, int nD) {
+__device__ __forceinline__ void face_gather(float* __restrict__ face, const float* __restrict__ inc, int nW, int nH,
+                                            int nD, int t) {
     const int fx = nW + (AXIS == 0), fy = nH + (AXIS == 1), fz = nD + (AXIS == 2);
-    const int t = blockIdx.x * BS + threadIdx.x;
     if (t >= fx * fy * fz) return;
     const int i = t % fx, j = (t / fx) % fy, k = t / (fx * fy);
     const int f = AXIS == 0 ? i : (AXIS == 1 ? j : k);
@@ -168,6 +167,19 @@ __global__ void __launch_bounds__(BS) k_face_gather(float* __restrict__ face, co
     if (lo) v = v + inc[c - sA];
     if (hi) v = v + inc[c];
     face[t] = v;
+}
+
+// the three axes' faces in one launch: inc is U's plane of increments, V's and
+// W's follow
+template <bool RANGE2>
+__global__ void __launch_bounds__(BS) k_face_gather(float* __restrict__ U, float* __restrict__ V,
+                                                    float* __restrict__ W, const float* __restrict__ inc, int nW,
+                                                    int nH, int nD, int firstV, int firstW) {
+    const int b = (int)blockIdx.x, t = (int)threadIdx.x;
+    const size_t N = (size_t)nW * nH * nD;
+    if (b < firstV) face_gather<0, RANGE2>(U, inc, nW, nH, nD, b * (int)BS + t);
+    else if (b < firstW) face_gather<1, RANGE2>(V, inc + N, nW, nH, nD, (b - firstV) * (int)BS + t);
+    else face_gather<2, RANGE2>(W, inc + 2 * N, nW, nH, nD, (b - firstW) * (int)BS + t);
 }
 
 // add_wind_kernel :337-390, restricted to the border slabs it touches
@@ -321,17 +333,17 @@ int launch_buoyancy_multi(hipStream_t st, bool mul, const BuoyJob* tab, int n, i
 }
 
 static int gather3(Solver& s, bool range2) {
-    const size_t N = (size_t)s.W * s.H * s.D;
-    const float* inc = s.tmp + 4 * N;
-    if (range2) {
-        LAUNCH((k_face_gather<0, true>), s.f[F_U].count(), s.f[F_U].front(), inc, s.W, s.H, s.D);
-        LAUNCH((k_face_gather<1, true>), s.f[F_V].count(), s.f[F_V].front(), inc + N, s.W, s.H, s.D);
-        LAUNCH((k_face_gather<2, true>), s.f[F_W].count(), s.f[F_W].front(), inc + 2 * N, s.W, s.H, s.D);
-    } else {
-        LAUNCH((k_face_gather<0, false>), s.f[F_U].count(), s.f[F_U].front(), inc, s.W, s.H, s.D);
-        LAUNCH((k_face_gather<1, false>), s.f[F_V].count(), s.f[F_V].front(), inc + N, s.W, s.H, s.D);
-        LAUNCH((k_face_gather<2, false>), s.f[F_W].count(), s.f[F_W].front(), inc + 2 * N, s.W, s.H, s.D);
-    }
+    const float* inc = s.tmp + 4 * (size_t)s.W * s.H * s.D;
+    const unsigned nu = blocks_for(s.f[F_U].count(), BS), nv = nu + blocks_for(s.f[F_V].count(), BS),
+                   nw = nv + blocks_for(s.f[F_W].count(), BS);
+    float *U = s.f[F_U].front(), *V = s.f[F_V].front(), *W = s.f[F_W].front();
+    if (range2)
+        hipLaunchKernelGGL(k_face_gather<true>, dim3(nw), dim3(BS), 0, s.stream, U, V, W, inc, s.W, s.H, s.D, (int)nu,
+                           (int)nv);
+    else
+        hipLaunchKernelGGL(k_face_gather<false>, dim3(nw), dim3(BS), 0, s.stream, U, V, W, inc, s.W, s.H, s.D, (int)nu,
+                           (int)nv);
+    BLZ_HIP(hipGetLastError());
     return BLZ_OK;
 }
 
