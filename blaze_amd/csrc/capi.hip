@@ -419,8 +419,10 @@ int Solver::project_solve(float dt_) {
 }
 
 int Solver::run_stage(int stage, float time, float dt_) {
-    int e0 = -1;
-    if (int e = span_begin(&e0)) return e;
+    int e0 = chain_ev;
+    chain_ev = -1;
+    if (e0 < 0)
+        if (int e = span_begin(&e0)) return e;
     int rc = BLZ_OK;
     switch (stage) {
     case BLZ_STAGE_COOLDOWN: rc = launch_cooldown(*this, dt_); break;
@@ -436,7 +438,9 @@ int Solver::run_stage(int stage, float time, float dt_) {
     default: set_error("unknown stage"); return BLZ_E_INVALID;
     }
     if (rc) return rc;
-    return span_end(stage, e0, 0);
+    if (int e = span_end(stage, e0, 0)) return e;
+    if (timing) chain_ev = spans.back().e1;
+    return BLZ_OK;
 }
 
 // FluidSolver::step, src/FluidSolver.cu:858-955 (stage gates :868-925)
@@ -480,12 +484,19 @@ int Solver::step_enqueue(float time, bool sync) {
         n = !(q >= 1.0f) ? 1 : (q > (float)s.max_substeps ? s.max_substeps : (int)q);
     }
     const float dts = dtf / (float)n;
+    // a stage begins where the one before it ends, the step with its first and
+    // last stage: one event for both (an event between two kernels costs the
+    // stream 2 to 4 us)
     int e0 = -1;
     if (int e = span_begin(&e0)) return e;
-    for (int q = 0; q < n; ++q)
-        if (int e = substep(time + (float)q * dts, dts)) return e;
+    chain_ev = e0;
+    int rc = BLZ_OK;
+    for (int q = 0; q < n && !rc; ++q) rc = substep(time + (float)q * dts, dts);
+    const int e1 = chain_ev;
+    chain_ev = -1;
+    if (rc) return rc;
     st.substeps = n;
-    if (int e = span_end(SPAN_STEP, e0, 0)) return e;
+    if (e1 >= 0) spans.push_back(Span{SPAN_STEP, e0, e1, 0, -1, -1, 0});
     if (int e = enqueue_solve_stats()) return e;
     if (sync) {
         BLZ_HIP(hipStreamSynchronize(stream));
@@ -678,7 +689,9 @@ int blz_run_stage(blz_solver* h, int stage, float time, float dt) {
     h->s.spans.clear();
     h->s.solves.clear();
     h->s.ev_used = 0;
-    if (int e = h->s.run_stage(stage, time, dt)) return e;
+    const int e = h->s.run_stage(stage, time, dt);
+    h->s.chain_ev = -1; // the caller may enqueue work of its own
+    if (e) return e;
     if (int e = h->s.enqueue_solve_stats()) return e;
     BLZ_HIP(hipStreamSynchronize(h->s.stream));
     return h->s.finalize();

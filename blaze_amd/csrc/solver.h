@@ -243,6 +243,7 @@ struct Solver {
     // from device memory instead of kernel arguments
     const float* dev_off = nullptr;
 
+    int chain_ev = -1; // a recorded event that the next stage's span may begin at (nothing enqueued since)
     int span_begin(int* e0);
     int span_end(int kind, int e0, int launches, int solve = -1, int batch = -1, int sweeps = 0);
     int resolve_spans();
