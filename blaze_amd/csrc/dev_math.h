@@ -127,7 +127,6 @@ __device__ __forceinline__ float trilinear_s(const Gv& g, const S& sc, f3 p) {
     if (gather_buffered(g)) return trilinear_g(g, gather_b(g), sc, p);
     return trilinear_g(g, GatherP{g.a}, sc, p);
 }
-__device__ __forceinline__ float trilinear(const Gv& g, float dx, f3 p) { return trilinear_s(g, DivDx{dx}, p); }
 
 // cerp / cerpc, src/Grid.h:148-163 (cubic Lagrange on nodes -1,0,1,2)
 __device__ __forceinline__ float cerp(float q0, float q1, float q2, float q3, float s) {
@@ -200,11 +199,6 @@ __device__ __forceinline__ float tricubic_s(const Gv& g, const S& sc, f3 p) {
     if (gather_buffered(g)) return tricubic_g<CLAMP>(g, gather_b(g), sc, p);
     return tricubic_g<CLAMP>(g, GatherP{g.a}, sc, p);
 }
-template <bool CLAMP>
-__device__ __forceinline__ float tricubic(const Gv& g, float dx, f3 p) {
-    return tricubic_s<CLAMP>(g, DivDx{dx}, p);
-}
-
 // fit, src/FluidSolver.cu:250-252
 __device__ __forceinline__ float fitf(float v, float minIn, float maxIn, float minOut, float maxOut) {
     return fmaxf(fminf((v - minIn) / (maxIn - minIn), 1.0f), 0.0f) * (maxOut - minOut) + minOut;
@@ -223,11 +217,12 @@ __device__ __forceinline__ uint32_t nhash(uint32_t s) {
     return s;
 }
 
-// saturating float -> uint32 (negative and NaN -> 0, >= 2^32 -> max)
+// saturating float -> uint32 (negative and NaN -> 0, >= 2^32 -> max), as the
+// conversion instruction does (C++ leaves those cases undefined)
 __device__ __forceinline__ uint32_t f2u_sat(float v) {
-    if (!(v > 0.0f)) return 0u;
-    if (v >= 4294967296.0f) return 0xffffffffu;
-    return (uint32_t)v;
+    uint32_t u;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(u) : "v"(v));
+    return u;
 }
 
 // randomIntGrid :120-123, float sum left to right
@@ -240,26 +235,14 @@ __device__ __forceinline__ uint32_t lattice_hash(float x, float y, float z, floa
     return nhash(f2u_sat(a));
 }
 
-// grad :179-201 (0xD = -y+z and 0xF = -y-z as in the source)
+// grad :179-201 (0xD = -y+z and 0xF = -y-z as in the source): two of the
+// coordinates, signed by the hash's low bits, without branches
+//   0-3: x y   4-7: x z   8-B: y z   C: y x   D: y z   E: y x   F: y z
 __device__ __forceinline__ float ngrad(uint32_t h, float x, float y, float z) {
-    switch (h & 0xFu) {
-    case 0x0: return x + y;
-    case 0x1: return -x + y;
-    case 0x2: return x - y;
-    case 0x3: return -x - y;
-    case 0x4: return x + z;
-    case 0x5: return -x + z;
-    case 0x6: return x - z;
-    case 0x7: return -x - z;
-    case 0x8: return y + z;
-    case 0x9: return -y + z;
-    case 0xA: return y - z;
-    case 0xB: return -y - z;
-    case 0xC: return y + x;
-    case 0xD: return -y + z;
-    case 0xE: return y - x;
-    default: return -y - z;
-    }
+    const uint32_t b = h & 0xFu;
+    const float p = b < 8u ? x : y;
+    const float q = b < 4u ? y : ((b & 0xDu) == 0xCu ? x : z);
+    return __uint_as_float(__float_as_uint(p) ^ (h << 31)) + __uint_as_float(__float_as_uint(q) ^ ((h >> 1) << 31));
 }
 
 __device__ __forceinline__ float nfade(float t) { return t * t * t * (t * (t * 6.0f - 15.0f) + 10.0f); }
