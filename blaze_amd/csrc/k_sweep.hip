@@ -28,7 +28,8 @@
 // us per sweep (times per launch / sweeps), one sweep per launch (the
 // autotuner's pick) -> here:
 //   32^3 7.1 -> 2.6, 64^3 10.8 -> 3.6, 90x75x62 12.0 -> 4.1, 96^3 15.0 ->
-//   5.8, 128^3 20.7 -> 6.9, 192^3 29.8 -> 15.2, 256^3 41.6 -> 20.4.
+//   5.8, 128^3 20.7 -> 6.9, 192^3 29.8 -> 13.9, 256^3 41.6 -> 18 (19 where
+//   checks every 10 sweeps cut them 3 + 3 + 2 + 2).
 #include "solver.h"
 
 namespace blz {
@@ -427,11 +428,14 @@ int go(hipStream_t st, const FusedScene* one, const FusedScene* tab, int n, int 
     return BLZ_OK;
 }
 
-// The tiles in use: columns and the most sweeps of a launch
+// The tiles in use: columns, the most sweeps of a launch, and how many are
+// usual. From 16x8 on two: three need two items per wave, and at 256^3 a launch
+// of three takes 57 us, one of two 35.
 struct Family {
-    int bx, by, tmax;
+    int bx, by, tmax, usual;
 };
-constexpr Family kFamilies[TILE_FAMILIES] = {{4, 4, 5}, {8, 4, 3}, {8, 8, 3}, {16, 16, 3}};
+constexpr Family kFamilies[TILE_FAMILIES] = {{4, 4, 5, 4},  {8, 4, 3, 3},  {8, 8, 3, 3},
+                                             {16, 8, 3, 2}, {16, 12, 3, 2}, {16, 16, 3, 2}};
 
 // T sweeps with a family's tiles, of one grid or of a table of grids
 int tile_sweeps(hipStream_t st, int family, int t, const FusedScene* one, const FusedScene* tab, int n, int blocks) {
@@ -444,8 +448,12 @@ int tile_sweeps(hipStream_t st, int family, int t, const FusedScene* one, const 
     case 13: return go<8, 4, 3, 1, 4>(st, one, tab, n, blocks);
     case 22: return go<8, 8, 2, 1, 4>(st, one, tab, n, blocks);
     case 23: return go<8, 8, 3, 1, 4>(st, one, tab, n, blocks);
-    case 32: return go<16, 16, 2, 1, 2>(st, one, tab, n, blocks);
-    case 33: return go<16, 16, 3, 2, 2>(st, one, tab, n, blocks);
+    case 32: return go<16, 8, 2, 1, 4>(st, one, tab, n, blocks);
+    case 33: return go<16, 8, 3, 2, 4>(st, one, tab, n, blocks);
+    case 42: return go<16, 12, 2, 1, 4>(st, one, tab, n, blocks);
+    case 43: return go<16, 12, 3, 2, 2>(st, one, tab, n, blocks);
+    case 52: return go<16, 16, 2, 1, 4>(st, one, tab, n, blocks);
+    case 53: return go<16, 16, 3, 2, 2>(st, one, tab, n, blocks);
     default: set_error("no such tile sweep"); return BLZ_E_INVALID;
     }
 }
@@ -471,6 +479,14 @@ Plan cut_into(int sweeps, int tmax) {
 }
 Plan plan_of(int family, int sweeps) {
     const int tmax = kFamilies[family].tmax;
+    if (kFamilies[family].usual == 2) { // launches of two, a few of three for what is left
+        Plan p;
+        p.launches = sweeps / 4 * 2;
+        p.shortest = 2;
+        p.longer = std::min(sweeps - 2 * p.launches, p.launches);
+        p.left = sweeps - 2 * p.launches - p.longer;
+        return p;
+    }
     const Plan p = cut_into(sweeps, tmax);
     if (tmax < 5) return p;
     // five sweeps in a launch need two items per wave: taken where they save
@@ -481,17 +497,20 @@ Plan plan_of(int family, int sweeps) {
     auto cost = [&](const Plan& q) {
         return (q.launches - q.longer) * us[q.shortest] + q.longer * us[q.shortest + 1] + 10.0 * q.left;
     };
-    const Plan q = cut_into(sweeps, 4);
+    const Plan q = cut_into(sweeps, kFamilies[family].usual);
     return cost(q) <= cost(p) ? q : p;
 }
 
 } // namespace
 
-// The tile for a W x H slab: the largest that still gives every CU (256) a
-// workgroup's worth of them, down to 4x4; a smaller tile has more rim to
-// compute again, a larger one leaves CUs idle. us per sweep of 4x4 / 8x4 /
-// 8x8 / 16x16 tiles: 64^3 3.6 / 4.0 / 4.4 / 6.8, 90x75x62 4.9 / 4.1 / 4.6 /
-// 6.9, 128^3 10.7 / 7.8 / 6.9 / 11.1, 192^3 31.8 / 19.2 / 17.6 / 15.2.
+// The tile for a W x H slab: the smallest of which every CU (256) gets at most
+// one; a smaller tile has more rim to compute again and takes turns, a larger
+// one leaves CUs idle. us per sweep of 4x4 / 8x4 / 8x8 / 16x16 tiles (all
+// with three sweeps per launch from 8x4 on): 64^3 3.6 / 4.0 / 4.4 / 6.8,
+// 90x75x62 4.9 / 4.1 / 4.6 / 6.9, 128^3 10.7 / 7.8 / 6.9 / 11.1. Of 8x8 /
+// 16x8 / 16x12 / 16x16 (8x8 with three, the others with two): 144^3 14.2 /
+// 10.0 / - / 13.1, 160^3 15.4 / 10.8 / - / 14.2, 192^3 25.7 / 16.8 / 13.9 /
+// 16.5, 256x128x256 22.1 / 15.4 / - / 20.7.
 int tile_family(int W, int H) {
     for (int f = 0; f < TILE_FAMILIES - 1; ++f)
         if (tile_count(f, W, H) <= 256) return f;

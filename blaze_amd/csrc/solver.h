@@ -280,7 +280,7 @@ bool fused_available(const Solver& s);
 // several sweeps per launch (k_sweep.hip): the tile family for a slab, its
 // tiles, and the launches of `sweeps` sweeps
 constexpr int VARIANT_TILES = 2000; // rbgs_variant: these sweeps
-constexpr int TILE_FAMILIES = 4;
+constexpr int TILE_FAMILIES = 6;
 int tile_family(int W, int H);
 int tile_count(int family, int W, int H);
 int launch_tile_sweeps(hipStream_t st, int family, const FusedScene* a, const FusedScene* b, int na, int blocks,

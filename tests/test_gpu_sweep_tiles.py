@@ -11,9 +11,9 @@ from helpers import compare, random_state, settings  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
-# 4x4 tiles up to 64x64 columns, then 8x4, 8x8 and 16x16
+# 4x4 tiles up to 64x64 columns, then 8x4, 8x8, 16x8, 16x12 and 16x16
 SHAPES = [(4, 4, 4), (6, 5, 9), (34, 33, 32), (64, 61, 6), (66, 90, 13), (90, 75, 5), (130, 66, 22), (122, 128, 8),
-          (162, 133, 7), (200, 98, 18)]
+          (162, 133, 7), (200, 98, 18), (200, 180, 7), (250, 220, 6)]
 
 
 def pair(s, st):
@@ -37,7 +37,8 @@ def test_tile_sweeps_bitwise(res, iters):
 
 
 @pytest.mark.parametrize("kind", ["tiny", "negzero", "decay", "inf"])
-@pytest.mark.parametrize("res", [(40, 36, 24), (90, 75, 10), (162, 133, 9)], ids=["4x4", "8x4", "16x16"])
+@pytest.mark.parametrize("res", [(40, 36, 24), (90, 75, 10), (162, 133, 9), (200, 180, 9), (250, 220, 9)],
+                         ids=["4x4", "8x4", "16x8", "16x12", "16x16"])
 def test_tile_sweeps_exact_division(kind, res):
     """Numerators outside the fast division's range in some lanes, groups or
     slabs only, and an infinity that spreads."""
