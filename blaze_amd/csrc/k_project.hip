@@ -1550,8 +1550,27 @@ FusedScene sweep_scene(const Solver& s, float dt, int src, int dst, const int* s
     return e;
 }
 
-// the sweeps of VARIANT_TILES on the planes home (through the spare ones),
-// the few left over as colour passes
+// VARIANT_TILES takes calls of four sweeps or more (launch_tile_sweeps makes
+// two launches of two sweeps or more); a pair of sweeps, or three, runs one
+// sweep per launch: row-pair sweeps with as many slab groups in flight as
+// divide a short column (us per sweep with 3 / 4 groups: 64x64x8 5.6 / 6.2,
+// 288x288x24 9.5 / 11.5, 256x256x16 9.4 / 8.0, 128^3 22.6 / 21.8, 256^3 44.2 /
+// 42.6), colour passes where the sweep's planes (12 bytes per cell) outgrow the
+// 256 MB Infinity Cache (320^3 90 against 110, 512x512x128 100 against 126).
+// Colour passes everywhere took 10.6 at 64x64x8, 25.0 at 128^3, 51.5 at 256^3.
+constexpr int TILE_MIN_SWEEPS = 4;
+static int variant_of(const Solver& s, int sweeps) {
+    int v = s.rbgs_variant ? s.rbgs_variant : s.rbgs_auto;
+    if (v == 0) v = 8;
+    if (v >= 100 && !fused_available(s)) v = 8;
+    if (v != VARIANT_TILES || sweeps >= TILE_MIN_SWEEPS) return v;
+    if (sweeps < 2) return 8;
+    if (12.0 * s.W * s.H * s.D > 256.0 * 1024 * 1024) return 4;
+    return s.L.Dg % 4 == 0 || s.L.Dg > 12 ? 1104 : 1103;
+}
+
+// the sweeps of VARIANT_TILES on the planes home (through the spare ones), an
+// odd one left over as colour passes
 static int tile_dispatch(Solver& s, float dt, int sweeps, const int* stop, int home, int* launches) {
     const int f = tile_family(s.W, s.H);
     const FusedScene to = sweep_scene(s, dt, home, 4, stop), back = sweep_scene(s, dt, 4, home, stop);
@@ -1569,7 +1588,7 @@ static int tile_dispatch(Solver& s, float dt, int sweeps, const int* stop, int h
 // last sweep as two colour passes; else two-pass sweeps in place
 int launch_rbgs_spare(Solver& s, float dt, int sweeps, const int* stop) {
     const float scale = (s.s.density * s.dx * s.dx) / dt;
-    const int v = s.rbgs_variant ? s.rbgs_variant : s.rbgs_auto;
+    const int v = variant_of(s, sweeps);
     if (s.judge_set == 6 && v == VARIANT_TILES) {
         int launches = 0;
         return tile_dispatch(s, dt, sweeps, stop, 6, &launches);
@@ -1583,9 +1602,7 @@ int launch_rbgs_spare(Solver& s, float dt, int sweeps, const int* stop) {
 
 int launch_rbgs_sweeps(Solver& s, float dt, int sweeps, const int* stop, int* launches, int* kind) {
     const float scale = (s.s.density * s.dx * s.dx) / dt; // Bridson p.75, :530
-    int v = s.rbgs_variant ? s.rbgs_variant : s.rbgs_auto;
-    if (v == 0) v = 8;
-    if (v >= 100 && !fused_available(s)) v = 8;
+    const int v = variant_of(s, sweeps);
     if (v == VARIANT_TILES) {
         *kind = 4;
         return tile_dispatch(s, dt, sweeps, stop, 0, launches);

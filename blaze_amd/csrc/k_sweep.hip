@@ -460,8 +460,8 @@ int tile_sweeps(hipStream_t st, int family, int t, const FusedScene* one, const 
 
 // How `sweeps` sweeps are cut into launches: an even number of them (home
 // planes -> spare -> home), as few as a family's longest launch allows, of
-// nearly equal lengths of two sweeps at least; what is left over (1, 2 or 3
-// sweeps, and one of 7 with three sweeps a launch) goes to the colour passes.
+// nearly equal lengths of two sweeps at least. Of four sweeps or more that
+// leaves at most one over (of 7, with three sweeps a launch), for the caller.
 struct Plan {
     int launches = 0, shortest = 0, longer = 0, left = 0; // `longer` launches have shortest + 1 sweeps
 };
@@ -522,7 +522,7 @@ int tile_count(int family, int W, int H) {
     return ((W + f.bx - 1) / f.bx) * ((H + f.by - 1) / f.by);
 }
 
-// `sweeps` sweeps less *left of them, alternately as a and as b say: the two
+// `sweeps` (four or more) less *left of them, alternately as a and as b say: the two
 // directions of one grid (na = 0) or of a table of na grids
 int launch_tile_sweeps(hipStream_t st, int family, const FusedScene* a, const FusedScene* b, int na, int blocks,
                        int sweeps, int* launches, int* left) {

@@ -1,7 +1,8 @@
 """Several sweeps per launch (the default sweeps, variant 2000) against the
 oracle bit for bit: every tile size the grid can get, one-column and clipped
-tiles at both rims, one to many slab groups (partly filled last groups), and
-sweep counts that leave one to three sweeps to the colour passes."""
+tiles at both rims, one to many slab groups (partly filled last groups), a
+sweep count that leaves one to the colour passes, and calls of fewer than four
+sweeps, which run one sweep per launch."""
 import numpy as np
 import pytest
 
@@ -33,7 +34,27 @@ def test_tile_sweeps_bitwise(res, iters):
     for x in (g, o):
         x.run_stage(B.STAGE_PRESSURE, 0.0, 1.0 / 24.0)
     compare("tile sweeps", g.field(B.FIELD_P), o.field(B.FIELD_P))
-    assert g.stats().rbgs_kernel == 4
+    assert g.stats().rbgs_kernel == (4 if iters >= 4 else 3)
+
+
+@pytest.mark.parametrize("every", [1, 2, 3])
+@pytest.mark.parametrize("res", [(18, 7, 4), (64, 61, 6), (90, 75, 22), (274, 258, 9), (40, 36, 52)],
+                         ids=lambda r: "x".join(map(str, r)))
+def test_calls_of_few_sweeps(res, every):
+    """Two or three sweeps between checks, or a cap of them: row-pair sweeps
+    (an odd one as colour passes), reported as such, whose launches are timed:
+    one per sweep and two per colour-passed sweep."""
+    print(f"[few sweeps] res={res} every={every}", flush=True)
+    s = settings(B, res, max_iter_solve=8, residual_tol=1e-30, residual_check_every=every)
+    g, o = pair(s, random_state(s, seed=every + sum(res)))
+    g.set_timing(True)
+    for x in (g, o):
+        x.run_stage(B.STAGE_PRESSURE, 0.0, 1.0 / 24.0)
+    st, batches = g.stats(), [every] * (8 // every) + [8 % every] * (8 % every > 0)
+    assert st.rbgs_iters_last == o.stats()["rbgs_iters_last"] == 8
+    assert st.rbgs_kernel == (1 if batches[-1] == 1 else 3)
+    assert st.rbgs_launches == sum(n + n % 2 for n in batches)
+    compare("few sweeps", g.field(B.FIELD_P), o.field(B.FIELD_P))
 
 
 @pytest.mark.parametrize("kind", ["tiny", "negzero", "decay", "inf"])
