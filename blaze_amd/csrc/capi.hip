@@ -315,19 +315,24 @@ int Solver::autotune(int sweeps, int* best, float* ms_per_sweep) {
     const int keep = rbgs_variant;
     int bestv = 8, rc = BLZ_OK, k = 0;
     float bestms = 1e30f;
+    const int call = s.residual_tol > 0.0f ? std::min(s.residual_check_every, s.max_iter_solve) : s.max_iter_solve;
     for (int v : cand) {
         if (v >= 100 && !fused_available(*this)) continue;
+        if (v == VARIANT_TILES && call < TILE_MIN_SWEEPS) continue; // such calls run one sweep per launch
         rbgs_variant = v;
+        // tiles: over as many sweeps as the solve runs at a time (10 to 20),
+        // after an untimed round of the same launches
+        const int count = v == VARIANT_TILES ? std::max(sweeps, std::clamp(call & ~1, 10, 20)) : sweeps;
         int launches = 0, kind = 0;
-        rc = launch_rbgs_sweeps(*this, dt, 2, zero_flag, &launches, &kind);
+        rc = launch_rbgs_sweeps(*this, dt, v == VARIANT_TILES ? count : 2, zero_flag, &launches, &kind);
         if (!rc) rc = hipEventRecord(e0, stream) == hipSuccess ? BLZ_OK : BLZ_E_HIP;
-        if (!rc) rc = launch_rbgs_sweeps(*this, dt, sweeps, zero_flag, &launches, &kind);
+        if (!rc) rc = launch_rbgs_sweeps(*this, dt, count, zero_flag, &launches, &kind);
         if (!rc) rc = hipEventRecord(e1, stream) == hipSuccess ? BLZ_OK : BLZ_E_HIP;
         if (!rc) rc = hipEventSynchronize(e1) == hipSuccess ? BLZ_OK : BLZ_E_HIP;
         if (rc) break;
         float ms = 0.0f;
         (void)hipEventElapsedTime(&ms, e0, e1);
-        ms /= (float)sweeps;
+        ms /= (float)count;
         if (ms_per_sweep && v != VARIANT_TILES) ms_per_sweep[k] = ms;
         ++k;
         if (ms < bestms) {

@@ -1550,7 +1550,7 @@ FusedScene sweep_scene(const Solver& s, float dt, int src, int dst, const int* s
     return e;
 }
 
-// VARIANT_TILES takes calls of four sweeps or more (launch_tile_sweeps makes
+// VARIANT_TILES takes calls of TILE_MIN_SWEEPS or more (launch_tile_sweeps makes
 // two launches of two sweeps or more); a pair of sweeps, or three, runs one
 // sweep per launch: row-pair sweeps with as many slab groups in flight as
 // divide a short column (us per sweep with 3 / 4 groups: 64x64x8 5.6 / 6.2,
@@ -1558,7 +1558,6 @@ FusedScene sweep_scene(const Solver& s, float dt, int src, int dst, const int* s
 // 42.6), colour passes where the sweep's planes (12 bytes per cell) outgrow the
 // 256 MB Infinity Cache (320^3 90 against 110, 512x512x128 100 against 126).
 // Colour passes everywhere took 10.6 at 64x64x8, 25.0 at 128^3, 51.5 at 256^3.
-constexpr int TILE_MIN_SWEEPS = 4;
 static int variant_of(const Solver& s, int sweeps) {
     int v = s.rbgs_variant ? s.rbgs_variant : s.rbgs_auto;
     if (v == 0) v = 8;

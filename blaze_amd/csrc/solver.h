@@ -281,6 +281,7 @@ bool fused_available(const Solver& s);
 // tiles, and the launches of `sweeps` sweeps
 constexpr int VARIANT_TILES = 2000; // rbgs_variant: these sweeps
 constexpr int TILE_FAMILIES = 6;
+constexpr int TILE_MIN_SWEEPS = 4;  // of a call; fewer run one sweep per launch
 int tile_family(int W, int H);
 int tile_count(int family, int W, int H);
 int launch_tile_sweeps(hipStream_t st, int family, const FusedScene* a, const FusedScene* b, int na, int blocks,

@@ -207,11 +207,12 @@ int blz_set_timing(blz_solver* h, int on);
    bits). */
 int blz_set_rbgs_variant(blz_solver* h, int variant);
 /* Autotuner (no reference counterpart): time `sweeps` sweeps of every
-   variant above on this grid (pressure restored afterwards) and keep the
-   fastest; ms_per_sweep (optional, 17 entries) receives the time of each
-   but 2000, in the order 2, 4, 8, 102, 103, 202, 203, 402, 403, 1103, 1104, 1105, 1106,
-   1203, 1204, 1403, 1404 (fused ones skipped when the spare planes do not
-   exist). */
+   variant above on this grid (pressure restored afterwards; 2000 over the
+   sweeps that a solve runs at a time, 10 to 20, and left out where those are
+   fewer than four) and keep the fastest; ms_per_sweep (optional, 17 entries)
+   receives the time of each but 2000, in the order 2, 4, 8, 102, 103, 202,
+   203, 402, 403, 1103, 1104, 1105, 1106, 1203, 1204, 1403, 1404 (fused ones
+   skipped when the spare planes do not exist). */
 int blz_autotune_rbgs(blz_solver* h, int sweeps, int* variant, float* ms_per_sweep);
 
 /* Change the pressure solve's limits of a live handle (no reference

@@ -57,6 +57,20 @@ def test_calls_of_few_sweeps(res, every):
     compare("few sweeps", g.field(B.FIELD_P), o.field(B.FIELD_P))
 
 
+@pytest.mark.parametrize("sweeps", [2, 20])
+def test_autotune_times_tile_sweeps(sweeps):
+    """However few sweeps the tuner is asked to time, the tiles are timed as a
+    solve runs them (at 128^3 they take under half of any other variant's
+    time); a solve that checks every two sweeps cannot use them."""
+    for every, want in ((10, True), (2, False)):
+        s = settings(B, (128, 128, 128), max_iter_solve=20, residual_tol=1e-30, residual_check_every=every)
+        g = B.Solver(s)
+        v, times = g.autotune(sweeps)
+        print(f"[tiles-autotune] {sweeps} sweeps, checks every {every}: {v} {times}", flush=True)
+        assert len(times) == 17
+        assert (v == 2000) == want
+
+
 @pytest.mark.parametrize("kind", ["tiny", "negzero", "decay", "inf"])
 @pytest.mark.parametrize("res", [(40, 36, 24), (90, 75, 10), (162, 133, 9), (200, 180, 9), (250, 220, 9)],
                          ids=["4x4", "8x4", "16x8", "16x12", "16x16"])
