@@ -291,7 +291,8 @@ void clear_step_stats(blz_stats& st) {
 
 // Time `sweeps` sweeps of every RBGS variant on the solver's rhs with the
 // pressure set to 1.0 (the pressure is restored afterwards; all variants
-// give the same bits); *best = the fastest. Synchronises the stream.
+// give the same bits); *best = the fastest, rbgs_one = the fastest that runs
+// one sweep per launch. Synchronises the stream.
 int Solver::autotune(int sweeps, int* best, float* ms_per_sweep) {
     // the one-sweep variants (reported), then several sweeps per launch
     static const int cand[] = {2,    4,    8,    102,  103,  202,  203,  402,  403,
@@ -313,9 +314,9 @@ int Solver::autotune(int sweeps, int* best, float* ms_per_sweep) {
     BLZ_HIP(hipEventCreate(&e0));
     BLZ_HIP(hipEventCreate(&e1));
     const int keep = rbgs_variant;
-    int bestv = 8, rc = BLZ_OK, k = 0;
+    int bestv = 8, one = 8, rc = BLZ_OK, k = 0;
     float bestms = 1e30f;
-    const int call = s.residual_tol > 0.0f ? std::min(s.residual_check_every, s.max_iter_solve) : s.max_iter_solve;
+    const int call = sweeps_per_call();
     for (int v : cand) {
         if (v >= 100 && !fused_available(*this)) continue;
         if (v == VARIANT_TILES && call < TILE_MIN_SWEEPS) continue; // such calls run one sweep per launch
@@ -338,6 +339,7 @@ int Solver::autotune(int sweeps, int* best, float* ms_per_sweep) {
         if (ms < bestms) {
             bestms = ms;
             bestv = v;
+            if (v != VARIANT_TILES) one = v; // the tiles come last
         }
     }
     rbgs_variant = keep;
@@ -350,6 +352,36 @@ int Solver::autotune(int sweeps, int* best, float* ms_per_sweep) {
         return rc;
     }
     *best = bestv;
+    rbgs_one = one;
+    return BLZ_OK;
+}
+
+// the most sweeps that a solve runs between two checks
+int Solver::sweeps_per_call() const {
+    return s.residual_tol > 0.0f ? std::min(s.residual_check_every, s.max_iter_solve) : s.max_iter_solve;
+}
+
+// The variant when none is set: several sweeps per launch, unless the spare
+// planes do not exist or the slab is both wide (more than one 16x16 tile per
+// CU) and flat (fewer than 8 groups of four slabs). There the steps that fill
+// and drain a launch, five of Dg + 5, weigh most, and the autotuner picks at
+// the first solve. us per sweep of the best
+// one-sweep variant / tiles at 10 sweeps per call: 2048x2048x8 140 / 205,
+// 1024x1024x8 31 / 46, 512x512x8 9.7 / 12.4, 1024x1024x24 69 / 78,
+// 288x288x24 8.4 / 9.0; beyond the line 1024x1024x32 110 / 93, 768x768x32
+// 50 / 45, 384x384x32 14.7 / 14.6, 320^3 90 / 68, 512^3 388 / 231; with a tile
+// per CU or fewer 64x64x4 4.8 / 2.5, 256x256x8 6.0 / 4.2, 256^3 41 / 25.
+// On a wide slab the autotuner also picks the variant of two- and three-sweep
+// calls: the rule for the others (variant_of) is up to 40% off there.
+int Solver::choose_variant() {
+    const bool wide = tile_count(TILE_FAMILIES - 1, W, H) > 256;
+    if (rbgs_auto == 0 && fused_available(*this) && !(wide && L.Dg < 8)) rbgs_auto = VARIANT_TILES;
+    const int call = sweeps_per_call();
+    const bool tune_one = rbgs_auto == VARIANT_TILES && wide && call > 1 && call < TILE_MIN_SWEEPS && rbgs_one == 0;
+    if (rbgs_auto != 0 && !tune_one) return BLZ_OK;
+    int best = 0;
+    if (int e = autotune(10, &best, nullptr)) return e;
+    if (rbgs_auto == 0) rbgs_auto = best;
     return BLZ_OK;
 }
 
@@ -365,13 +397,8 @@ int Solver::autotune(int sweeps, int* best, float* ms_per_sweep) {
 // its result after the step.
 int Solver::project_solve(float dt_) {
     const int cap = s.max_iter_solve;
-    // variant 0: several sweeps per launch (faster than every one-sweep
-    // variant on all grids measured, 32^3 .. 256^3); without spare planes
-    // the autotuner's choice for this grid, made at the first solve
-    if (rbgs_variant == 0 && rbgs_auto == 0 && cap > 0) {
-        if (fused_available(*this)) rbgs_auto = VARIANT_TILES;
-        else if (int e = autotune(10, &rbgs_auto, nullptr)) return e;
-    }
+    if (rbgs_variant == 0 && cap > 0)
+        if (int e = choose_variant()) return e;
     const int q = (int)solves.size();
     if (q >= MAX_SOLVES) {
         set_error("too many pressure solves enqueued without synchronisation");

@@ -1502,8 +1502,7 @@ bool fused_available(const Solver& s) { return s.prb_floats >= 6 * s.Np; }
 // per block, g = 2, 3 groups in flight) = fused sweeps in pairs, an odd
 // last sweep as two colour passes; 1000 + 100*w + g (g = 3..6) = the same
 // with the row-pair fused sweep; VARIANT_TILES = several sweeps per launch;
-// 0 = VARIANT_TILES, or the autotuner's choice where the spare planes do not
-// exist (8 where it has not run).
+// 0 = Solver::choose_variant's (8 where no solve has run).
 bool rbgs_variant_valid(int v) {
     return v == 0 || v == VARIANT_TILES || v == 2 || v == 4 || v == 8 || v == 102 || v == 103 || v == 202 || v == 203 || v == 402 ||
            v == 403 || v == 1103 || v == 1104 || v == 1105 || v == 1106 || v == 1203 || v == 1204 || v == 1403 ||
@@ -1552,18 +1551,20 @@ FusedScene sweep_scene(const Solver& s, float dt, int src, int dst, const int* s
 
 // VARIANT_TILES takes calls of TILE_MIN_SWEEPS or more (launch_tile_sweeps makes
 // two launches of two sweeps or more); a pair of sweeps, or three, runs one
-// sweep per launch: row-pair sweeps with as many slab groups in flight as
-// divide a short column (us per sweep with 3 / 4 groups: 64x64x8 5.6 / 6.2,
-// 288x288x24 9.5 / 11.5, 256x256x16 9.4 / 8.0, 128^3 22.6 / 21.8, 256^3 44.2 /
-// 42.6), colour passes where the sweep's planes (12 bytes per cell) outgrow the
-// 256 MB Infinity Cache (320^3 90 against 110, 512x512x128 100 against 126).
-// Colour passes everywhere took 10.6 at 64x64x8, 25.0 at 128^3, 51.5 at 256^3.
+// sweep per launch: the autotuner's pick, if it ran, else row-pair sweeps with
+// as many slab groups in flight as divide a short column (us per sweep with
+// 3 / 4 groups: 64x64x8 5.6 / 6.2, 288x288x24 9.5 / 11.5, 256x256x16 9.4 /
+// 8.0, 128^3 22.6 / 21.8, 256^3 44.2 / 42.6), colour passes where the sweep's
+// planes (12 bytes per cell) outgrow the 256 MB Infinity Cache (320^3 90
+// against 110, 512x512x128 100 against 126). Colour passes everywhere took
+// 10.6 at 64x64x8, 25.0 at 128^3, 51.5 at 256^3.
 static int variant_of(const Solver& s, int sweeps) {
     int v = s.rbgs_variant ? s.rbgs_variant : s.rbgs_auto;
     if (v == 0) v = 8;
     if (v >= 100 && !fused_available(s)) v = 8;
     if (v != VARIANT_TILES || sweeps >= TILE_MIN_SWEEPS) return v;
     if (sweeps < 2) return 8;
+    if (s.rbgs_one) return s.rbgs_one;
     if (12.0 * s.W * s.H * s.D > 256.0 * 1024 * 1024) return 4;
     return s.L.Dg % 4 == 0 || s.L.Dg > 12 ? 1104 : 1103;
 }
@@ -1609,7 +1610,7 @@ int launch_rbgs_sweeps(Solver& s, float dt, int sweeps, const int* stop, int* la
     if (v >= 100) {
         const int pairs = sweeps / 2;
         *launches = 2 * pairs + 2 * (sweeps & 1);
-        *kind = v >= 1000 ? 3 : 2;
+        *kind = pairs == 0 ? 1 : (v >= 1000 ? 3 : 2);
         if (int e = fused_dispatch(s, v, scale, pairs, stop)) return e;
         return (sweeps & 1) ? rbgs_passes<8>(s, scale, 1, stop) : BLZ_OK;
     }

@@ -225,8 +225,9 @@ struct Solver {
     std::vector<hipEvent_t> evpool;
     size_t ev_used = 0;
     std::vector<Span> spans;
-    int rbgs_variant = 0; // requested variant (0 = VARIANT_TILES, or autotuned without spare planes)
+    int rbgs_variant = 0; // requested variant (0: choose_variant's)
     int rbgs_auto = 0;    // the variant used when rbgs_variant == 0
+    int rbgs_one = 0;     // VARIANT_TILES' calls of two or three sweeps: the autotuner's one-sweep variant, if it ran
     // learned warm start (attached network; activations of its own)
     const Net* ws_src = nullptr;
     Net* ws_net = nullptr;     // view: shares ws_src's weights, owns activations
@@ -259,6 +260,8 @@ struct Solver {
     int run_stage(int stage, float time, float dt);
     int project_solve(float dt);
     int autotune(int sweeps, int* best, float* ms_per_sweep);
+    int sweeps_per_call() const;
+    int choose_variant();
     int enqueue_solve_stats();
     int max_abs_velocity(float* out);
 };

@@ -202,9 +202,9 @@ int blz_set_timing(blz_solver* h, int on);
    x = 1/2/4 in 10x; 1x03 .. 1x06 = row-pair fused whole-sweep kernel (two
    rows per wave, 3 to 6 groups in flight, x = 1/2/4 waves per block);
    2000 = several sweeps per launch, tiles of columns chosen by the grid;
-   0 = default: 2000, or on grids too large for its spare planes the
-   autotuner's choice, made at the first solve (every variant gives the same
-   bits). */
+   0 = default: 2000, or on grids too large for its spare planes, or of fewer
+   than 29 slabs of more than 256 tiles of 16x16 cells, the autotuner's choice,
+   made at the first solve (every variant gives the same bits). */
 int blz_set_rbgs_variant(blz_solver* h, int variant);
 /* Autotuner (no reference counterpart): time `sweeps` sweeps of every
    variant above on this grid (pressure restored afterwards; 2000 over the

@@ -38,7 +38,7 @@ def test_tile_sweeps_bitwise(res, iters):
 
 
 @pytest.mark.parametrize("every", [1, 2, 3])
-@pytest.mark.parametrize("res", [(18, 7, 4), (64, 61, 6), (90, 75, 22), (274, 258, 9), (40, 36, 52)],
+@pytest.mark.parametrize("res", [(18, 7, 4), (64, 61, 6), (90, 75, 22), (256, 256, 9), (40, 36, 52)],
                          ids=lambda r: "x".join(map(str, r)))
 def test_calls_of_few_sweeps(res, every):
     """Two or three sweeps between checks, or a cap of them: row-pair sweeps
@@ -69,6 +69,26 @@ def test_autotune_times_tile_sweeps(sweeps):
         print(f"[tiles-autotune] {sweeps} sweeps, checks every {every}: {v} {times}", flush=True)
         assert len(times) == 17
         assert (v == 2000) == want
+
+
+@pytest.mark.parametrize("res,every,want", [((1024, 1024, 8), 10, (1, 2, 3)), ((1024, 1024, 8), 2, (1, 2, 3)),
+                                            ((274, 258, 33), 10, (4,)), ((274, 258, 33), 3, (1, 2, 3)),
+                                            ((512, 512, 88), 2, (1, 2, 3)), ((256, 256, 5), 10, (4,))],
+                         ids=["flat", "flat-2", "wide", "wide-3", "large-2", "tile-per-CU"])
+def test_default_sweeps_of_wide_slabs(res, every, want):
+    """More than one 16x16 tile per CU: the tiles, except on few slabs, where
+    a launch's filling and draining steps cost more than they save (1.5 times
+    the best one-sweep variant's time at 1024x1024x8)."""
+    print(f"[tiles-wide] res={res} every={every}", flush=True)
+    s = settings(B, res, max_iter_solve=every, residual_tol=1e-30, residual_check_every=every)
+    rng = np.random.default_rng(every)
+    W, H, D = res
+    st = {w: rng.random((D, H, W), dtype=np.float32) - np.float32(0.5) for w in (B.FIELD_P, B.FIELD_RHS)}
+    g, o = pair(s, st)
+    for x in (g, o):
+        x.run_stage(B.STAGE_PRESSURE, 0.0, 1.0 / 24.0)
+    assert g.stats().rbgs_kernel in want
+    compare("wide slab", g.field(B.FIELD_P), o.field(B.FIELD_P))
 
 
 @pytest.mark.parametrize("kind", ["tiny", "negzero", "decay", "inf"])
