@@ -23,6 +23,7 @@
 // transmittance, and both marches stop after 65536 samples.
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "solver.h"
 
@@ -30,9 +31,6 @@ namespace blz {
 
 namespace {
 
-constexpr int RT = 2;       // pixels per tile side
-constexpr int PX = RT * RT;  // pixels per tile
-constexpr int SPW = 64 / PX; // samples of each ray that a wave takes
 constexpr int RES_STEP = 8; // frames are multiples of the reference's 8x8 launch tiles
 constexpr int MAX_MARCH = 1 << 16;
 
@@ -87,21 +85,25 @@ __device__ __forceinline__ Texel texel_at(int nx, int ny, int nz, V3 g) {
 
 typedef float f2a4 __attribute__((ext_vector_type(2), aligned(4)));
 
-// The two texels of a row come as one 8-byte load (the pair moved inside the
-// row at its ends); WIDE: volumes of 4 GiB and more, whose byte offsets do
-// not fit 32 bits.
-template <bool WIDE>
+// PAIR: the two texels of a row as one 8-byte load (the pair moved inside the
+// row at its ends), where a wave's lanes are spread along rays. Lanes beside
+// each other in the image read beside each other, and there the eight 4-byte
+// loads take half the time: 1920x1080 through a full 256^3, one light, 8.6 ms
+// against 11.3. WIDE: volumes of 4 GiB and more, whose byte offsets do not fit
+// 32 bits.
+template <bool WIDE, bool PAIR>
 __device__ __forceinline__ float tex_lin(const float* __restrict__ v, int nx, int ny, int nz, const Texel& q) {
     const int ya = min(max(q.j, 0), ny - 1), yc = min(max(q.j + 1, 0), ny - 1);
     const int za = min(max(q.k, 0), nz - 1), zc = min(max(q.k + 1, 0), nz - 1);
-    const int x = min(max(q.i, 0), max(nx - 2, 0));
+    const int x = min(max(q.i, 0), max(nx - 2, 0)), xa = min(max(q.i, 0), nx - 1), xc = min(max(q.i + 1, 0), nx - 1);
     const bool low = q.i < 0, high = q.i >= nx - 1;
+    auto at = [&](int i, int j, int k) {
+        if (WIDE) return v + ((size_t)k * ny + j) * nx + i;
+        return (const float*)((const char*)v + (unsigned)((k * ny + j) * nx + i) * 4u);
+    };
     auto row = [&](int j, int k) {
-        const float* p;
-        if (WIDE)
-            p = v + ((size_t)k * ny + j) * nx + x;
-        else
-            p = (const float*)((const char*)v + (unsigned)((k * ny + j) * nx + x) * 4u);
+        if (!PAIR) return (1.0f - q.a) * *at(xa, j, k) + q.a * *at(xc, j, k);
+        const float* p = at(x, j, k);
         if (nx < 2) return (1.0f - q.a) * p[0] + q.a * p[0]; // uniform
         const f2a4 t = *(const f2a4*)p;
         return (1.0f - q.a) * (high ? t[1] : t[0]) + q.a * (low ? t[0] : t[1]);
@@ -359,9 +361,9 @@ __device__ __forceinline__ bool occupied(const unsigned* bits, const Occ& o, con
 }
 
 // transmittance from `pos` to a light: SU samples at a time, so that their
-// loads overlap (the exponentials still follow each other)
-constexpr int SU = 2;
-template <class S, bool WIDE>
+// loads overlap (the exponentials still follow each other); BITS: samples in
+// clear bricks are passed over
+template <int SU, bool BITS, bool PAIR, class S, bool WIDE>
 __device__ __forceinline__ V3 shadow_march(const float* __restrict__ T, const unsigned* bits, const RScene& s,
                                            const S& sc, const Occ& o, V3 lo, V3 hi, V3 pos, V3 dir) {
     V3 strans = mkv(1.0f, 1.0f, 1.0f);
@@ -380,7 +382,7 @@ __device__ __forceinline__ V3 shadow_march(const float* __restrict__ T, const un
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
             q[u] = texel_at(s.W, s.H, s.D, w2g(s, sc, sr.o + st * sr.d));
-            take[u] = st <= end && m + u < MAX_MARCH && occupied(bits, o, s, q[u]);
+            take[u] = st <= end && m + u < MAX_MARCH && (!BITS || occupied(bits, o, s, q[u]));
             any |= take[u];
             at[u] = st;
             st += s.s_step;
@@ -389,7 +391,7 @@ __device__ __forceinline__ V3 shadow_march(const float* __restrict__ T, const un
         float sd[SU];
 #pragma unroll
         for (int u = 0; u < SU; ++u)
-            sd[u] = tex_lin<WIDE>(T, s.W, s.H, s.D, q[u]) * s.density_scale * s.shadow_density_scale;
+            sd[u] = tex_lin<WIDE, PAIR>(T, s.W, s.H, s.D, q[u]) * s.density_scale * s.shadow_density_scale;
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
             if (!take[u] || sd[u] < s.cutoff) continue;
@@ -405,8 +407,42 @@ __device__ __forceinline__ V3 shadow_march(const float* __restrict__ T, const un
     return strans;
 }
 
-// render_kernel: a workgroup of RW waves per 2x2 pixels. Along a ray only the
-// transmittance is a chain, and it needs the densities alone; so the tile
+// a sample's emission (render_kernel :190-203)
+template <bool PAIR, bool WIDE>
+__device__ __forceinline__ V3 emission_at(const float* __restrict__ scat, const RScene& s, V3 g, float temp) {
+    if (!(s.emission_scale > 0.0f)) return mkv(0.0f, 0.0f, 0.0f);
+    const float scatter = tex_lin<WIDE, PAIR>(
+        scat, s.Ws, s.Hs, s.Ds, texel_at(s.Ws, s.Hs, s.Ds, mkv(g.x / 4.0f, g.y / 4.0f, g.z / 4.0f)));
+    return ramp_color(s, temp) * s.emission_scale +
+           s.ms_color * scatter * s.ms_scale * smoothstep_f(s.ms_mask_a, s.ms_mask_b, temp);
+}
+
+// the camera ray of pixel (i, j): Camera::getRay, normalize(top_left +
+// u*horizontal + v*vertical - origin)
+__device__ __forceinline__ Ray camera_ray(const RScene& s, int i, int j) {
+    const V3 q = s.top_left + (((float)i + 0.5f) / s.res_x) * s.horizontal +
+                 (((float)j + 0.5f) / s.res_y) * s.vertical - s.origin;
+    const float inv_len = 1.0f / sqrtf(q.x * q.x + q.y * q.y + q.z * q.z);
+    return make_ray(s.origin, q * inv_len);
+}
+
+// the box of the bricks that are not clear, and a camera ray's part in it
+struct Box {
+    V3 lo, hi;
+};
+__device__ __forceinline__ Box brick_box(const unsigned* __restrict__ occ, const Occ& o) {
+    const float inf = __int_as_float(0x7f800000);
+    const float* b = (const float*)(occ + o.words);
+    if (!o.box) return Box{mkv(-inf, -inf, -inf), mkv(inf, inf, inf)};
+    return Box{mkv(b[0], b[1], b[2]), mkv(b[3], b[4], b[5])};
+}
+__device__ __forceinline__ Span camera_span(const Ray& r, const Box& box, const RScene& s, const Occ& o) {
+    return box_span(r, box.lo, box.hi,
+                    o.margin_dom + o.margin * (fabsf(s.origin.x) + fabsf(s.origin.y) + fabsf(s.origin.z)));
+}
+
+// render_kernel: a workgroup of RW waves per RT x RT pixels. Along a ray only
+// the transmittance is a chain, and it needs the densities alone; so the tile
 // takes up to SPW RW samples of its rays at a time, a thread per sample (a
 // wave: SPW samples of every ray, neighbours in space). Each thread has its
 // sample's density, emission and exp; each wave runs the chain; the waves draw
@@ -414,41 +450,38 @@ __device__ __forceinline__ V3 shadow_march(const float* __restrict__ T, const un
 // sample's light; and wave 0 adds it up in the reference's order while the
 // other starts on the next samples. Rays are cut to the box of the bricks that
 // are not clear, and samples in clear bricks read nothing. Bound by the vector
-// instructions of the shadow marches (45 of 64 lanes, 84% of the CUs busy).
+// instructions of the shadow marches. Small tiles spread the few heavy rays of
+// a small frame over the chip; each lane walks its ray's chain of SPW RW
+// samples, so large tiles do less of it. Which frame gets which:
+// render_with.
 //
-// 640x360 over 256^3, three lights, gas in 4% of the pixels: one wave per 8x8
-// tile that marches alone took 9.9 ms, the heaviest tiles last; eight waves
-// per 8x8 tile 1.48 ms, 4x4 tiles with four waves 1.09, the rays cut to the
-// box about 0.8, and 2x2 tiles with two waves 0.70 (one wave: 0.80, four with
-// 64 samples at a time: 1.1; SU = 1: 0.75).
+// The kernel over 256^3 at 640x360, three lights, gas in 4% of the pixels: one
+// wave per 8x8 tile that marches alone took 9.9 ms, the heaviest tiles last;
+// 2x2 tiles 0.70 (one wave: 0.80, four with 64 samples at a time: 1.1; SU = 1:
+// 0.75).
 constexpr int RW = 2, RTASKS = 10;
-template <class S, bool WIDE>
+template <int RT, bool PAIR, class S, bool WIDE>
 __global__ void __launch_bounds__(RW * 64) k_render(const float* __restrict__ T, const float* __restrict__ scat,
                                                     const unsigned* __restrict__ occ, float* __restrict__ fb,
                                                     RScene s, S sc, Occ o, int groups) {
+    constexpr int PX = RT * RT;  // pixels of a tile
+    constexpr int SPW = 64 / PX; // samples of each ray that a wave takes
+    static_assert(3 * PX <= 64, "wave 0 has a lane per channel and pixel");
     __shared__ unsigned bits[OCC_WORDS];
     __shared__ unsigned long long act[2][RW];
-    // [group of four samples][lane]
+    // [group of SPW samples of each ray][lane]
     __shared__ float s_pt[RW][64], s_dT[3][RW][64], s_em[3][RW][64], s_str[RTASKS][3][64];
     __shared__ int next;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int px = lane % PX;
     const int i = blockIdx.x * RT + px % RT, j = blockIdx.y * RT + px / RT;
     for (int t = threadIdx.x; t < o.words; t += RW * 64) bits[t] = occ[t];
-    // Camera::getRay: normalize(top_left + u*horizontal + v*vertical - origin)
-    const V3 q = s.top_left + (((float)i + 0.5f) / s.res_x) * s.horizontal +
-                 (((float)j + 0.5f) / s.res_y) * s.vertical - s.origin;
-    const float inv_len = 1.0f / sqrtf(q.x * q.x + q.y * q.y + q.z * q.z);
-    Ray pr = make_ray(s.origin, q * inv_len);
+    Ray pr = camera_ray(s, i, j);
     bool alive = box_hit(pr, s.dom_min, s.dom_max);
     V3 trans = mkv(1.0f, 1.0f, 1.0f);
     const V3 one = mkv(1.0f, 1.0f, 1.0f);
-    const V3 inf3 = one * __int_as_float(0x7f800000);
-    const float* box = (const float*)(occ + o.words);
-    const V3 lo = o.box ? mkv(box[0], box[1], box[2]) : -1.0f * inf3, hi = o.box ? mkv(box[3], box[4], box[5]) : inf3;
-    const Span span =
-        box_span(pr, lo, hi,
-                 o.margin_dom + o.margin * (fabsf(s.origin.x) + fabsf(s.origin.y) + fabsf(s.origin.z)));
+    const Box box = brick_box(occ, o);
+    const Span span = camera_span(pr, box, s, o);
     const float end = span.t1 < pr.t1 ? span.t1 : pr.t1;
     float lumi = 0.0f; // of wave 0's lane (channel, pixel)
     const int rn = SPW * groups, ntask = groups * s.light_count;
@@ -473,17 +506,11 @@ __global__ void __launch_bounds__(RW * 64) k_render(const float* __restrict__ T,
             const Texel tq = texel_at(s.W, s.H, s.D, g);
             on = on && occupied(bits, o, s, tq);
             if (on) {
-                const float temp = tex_lin<WIDE>(T, s.W, s.H, s.D, tq);
+                const float temp = tex_lin<WIDE, PAIR>(T, s.W, s.H, s.D, tq);
                 const float dens = temp * s.density_scale;
                 on = !(dens < s.cutoff);
                 if (on) {
-                    if (s.emission_scale > 0.0f) {
-                        const float scatter =
-                            tex_lin<WIDE>(scat, s.Ws, s.Hs, s.Ds,
-                                          texel_at(s.Ws, s.Hs, s.Ds, mkv(g.x / 4.0f, g.y / 4.0f, g.z / 4.0f)));
-                        emission = ramp_color(s, temp) * s.emission_scale +
-                                   s.ms_color * scatter * s.ms_scale * smoothstep_f(s.ms_mask_a, s.ms_mask_b, temp);
-                    }
+                    emission = emission_at<PAIR, WIDE>(scat, s, g, temp);
                     dT = bexp3(s.extinction * dens * s.p_step);
                     s_pt[wv][lane] = from;
                     s_dT[0][wv][lane] = dT.x;
@@ -521,8 +548,8 @@ __global__ void __launch_bounds__(RW * 64) k_render(const float* __restrict__ T,
             if (t >= ntask) break;
             const int l = t / groups, w = t - l * groups;
             if (!((use >> (SPW * w + lane / PX)) & 1)) continue;
-            const V3 str = shadow_march<S, WIDE>(T, bits, s, sc, o, lo, hi, pr.o + s_pt[w][lane] * pr.d,
-                                                 -1.0f * s.light_dir[l]);
+            const V3 str = shadow_march<2, true, PAIR, S, WIDE>(T, bits, s, sc, o, box.lo, box.hi,
+                                                                pr.o + s_pt[w][lane] * pr.d, -1.0f * s.light_dir[l]);
             s_str[t][0][lane] = str.x;
             s_str[t][1][lane] = str.y;
             s_str[t][2][lane] = str.z;
@@ -556,6 +583,55 @@ __global__ void __launch_bounds__(RW * 64) k_render(const float* __restrict__ T,
         }
     }
     if (wv == 0 && lane < 3 * PX) fb[3 * ((size_t)i + (size_t)(int)s.res_x * j) + lane / PX] = lumi;
+}
+
+// A thread per pixel, 8x8 pixels per wave, each marching its ray and its
+// samples' shadow rays alone: the least work of all, and with enough waves on
+// every CU their unlike lengths even out. The bricks' bits cost more than they
+// save here; the box does not.
+//
+// 1920x1080 over 256^3 (steps of two cells), 2x2 and 4x4 tiles against this:
+// full of gas, one light 22 and 9.5 against 8.7 ms; one cell in a thousand,
+// three lights 14 and 4.4 against 3.0; gas in 4% of the pixels, one light 3.4
+// and 2.1 against 2.1.
+constexpr int PT = 8;
+template <class S, bool WIDE>
+__global__ void __launch_bounds__(PT * PT) k_render_px(const float* __restrict__ T, const float* __restrict__ scat,
+                                                       const unsigned* __restrict__ occ, float* __restrict__ fb,
+                                                       RScene s, S sc, Occ o) {
+    const int i = blockIdx.x * PT + threadIdx.x % PT, j = blockIdx.y * PT + threadIdx.x / PT;
+    const Ray pr = camera_ray(s, i, j);
+    V3 lumi = mkv(0.0f, 0.0f, 0.0f), trans = mkv(1.0f, 1.0f, 1.0f);
+    const V3 one = mkv(1.0f, 1.0f, 1.0f);
+    if (Ray r = pr; box_hit(r, s.dom_min, s.dom_max)) {
+        const Box box = brick_box(occ, o);
+        const Span span = camera_span(r, box, s, o);
+        const float end = span.t1 < r.t1 ? span.t1 : r.t1;
+        float pt = r.t0 + s.dx * 0.5f;
+        int n = 0;
+        for (; pt < span.t0 && pt <= end && n < MAX_MARCH; ++n) pt += s.p_step;
+        for (; pt <= end && n < MAX_MARCH; pt += s.p_step, ++n) {
+            const V3 pos = r.o + pt * r.d;
+            const V3 g = w2g(s, sc, pos);
+            const float temp = tex_lin<WIDE, false>(T, s.W, s.H, s.D, texel_at(s.W, s.H, s.D, g));
+            const float dens = temp * s.density_scale;
+            if (dens < s.cutoff) continue;
+            const V3 emission = emission_at<false, WIDE>(scat, s, g, temp);
+            const V3 dT = bexp3(s.extinction * dens * s.p_step);
+            for (int l = 0; l < s.light_count; ++l) {
+                const V3 str = shadow_march<1, false, false, S, WIDE>(T, nullptr, s, sc, o, box.lo, box.hi, pos,
+                                                                      -1.0f * s.light_dir[l]);
+                lumi = lumi + s.albedo * str * trans * s.light_illum[l] * (one - dT);
+            }
+            lumi = lumi + trans * emission * (one - dT);
+            trans = trans * dT;
+            if (sqlen(trans) < s.cutoff) break;
+        }
+    }
+    float* p = fb + 3 * ((size_t)i + (size_t)(int)s.res_x * j);
+    p[0] = lumi.x;
+    p[1] = lumi.y;
+    p[2] = lumi.z;
 }
 
 inline unsigned nblk(size_t n) { return (unsigned)((n + 255) / 256); }
@@ -710,22 +786,49 @@ static int render_with(Solver& s, const blz_render_settings& r, float* host_rgb,
     o.margin_dom = 2.0f * s.dx + 1e-5f * reach;
     if (o.box)
         hipLaunchKernelGGL(k_rnd_box, dim3(1), dim3(1024), 0, s.stream, occ, o, sc.dom_min, sc.dom_size, s.dx);
-    // groups of four samples per round: one per wave, fewer where the shadow
+    // groups of SPW samples per round: one per wave, fewer where the shadow
     // marches of more than RTASKS / RW lights need the room
     const int groups = std::min(RW, RTASKS / std::max(1, r.light_count));
-    const dim3 grid((unsigned)(r.width / RT), (unsigned)(r.height / RT)), block(RW * 64);
+    // The tile by the frame's pixels and lights. ms of a call with 2x2 tiles /
+    // 4x4 tiles / a thread per pixel over 256^3, with gas in 4% of the pixels,
+    // full of gas, and with one cell in a thousand:
+    //   64x64, 3 lights      0.51 / 0.76 / 5.0   1.8 / 3.0 / 25    1.3 / 1.7 / 11
+    //   320x184, 3 lights    0.55 / 0.82 / 4.3   6.9 / 10 / 24     2.5 / 1.8 / 12
+    //   320x184, none        0.27 / 0.25 / 0.33  0.47 / 0.38 / 0.46  0.39 / 0.32 / 0.46
+    //   640x360, 3 lights    1.03 / 0.94 / 3.8   21 / 12 / 24      4.5 / 2.2 / 6.1
+    //   640x360, none        0.48 / 0.40 / 0.44  1.2 / 0.71 / 0.64 0.84 / 0.57 / 0.55
+    //   1280x720, 3 lights   3.0 / 2.1 / 5.3     72 / 41 / 58      13 / 4.2 / 4.8
+    //   1280x720, 1 light    1.6 / 1.1 / 1.3     10 / 4.4 / 4.7    4.1 / 1.7 / 1.4
+    //   1920x1080, 3 lights  4.1 / 2.5 / 3.0     54 / 26 / 28      14 / 4.4 / 3.0
+    // Against the first build (a wave per 8x8 pixels alone) this rule took 0.04
+    // to 1.04 of the time on eleven volumes of 32^3 to 256^3 at 17 frame sizes;
+    // 2x2 tiles for all took up to 4.5 times as long (1920x1080 of the last).
+    const long long pixels = (long long)r.width * r.height;
+    const int tile = pixels >= 200000 + 500000ll * r.light_count ? PT
+                     : pixels >= (r.light_count ? 200000 : 30000) ? 4 : 2;
+    const dim3 grid((unsigned)(r.width / tile), (unsigned)(r.height / tile));
     const bool wide = (size_t)s.W * s.H * s.D >= ((size_t)1 << 30);
+    auto launch = [&](auto scale, auto w) {
+        using S = decltype(scale);
+        constexpr bool WIDE = decltype(w)::value;
+        if (tile == PT)
+            hipLaunchKernelGGL((k_render_px<S, WIDE>), grid, dim3(PT * PT), 0, s.stream, T, scat[0], occ, fb, sc,
+                               scale, o);
+        else if (tile == 4)
+            hipLaunchKernelGGL((k_render<4, false, S, WIDE>), grid, dim3(RW * 64), 0, s.stream, T, scat[0], occ, fb,
+                               sc, scale, o, groups);
+        else
+            hipLaunchKernelGGL((k_render<2, true, S, WIDE>), grid, dim3(RW * 64), 0, s.stream, T, scat[0], occ, fb,
+                               sc, scale, o, groups);
+    };
     float inv = 0.0f;
-#define RENDER(S, WIDE, sc_) \
-    hipLaunchKernelGGL((k_render<S, WIDE>), grid, block, 0, s.stream, T, scat[0], occ, fb, sc, sc_, o, groups)
     if (dx_pow2(s.dx, &inv)) {
-        if (wide) RENDER(MulDx, true, MulDx{inv});
-        else RENDER(MulDx, false, MulDx{inv});
+        if (wide) launch(MulDx{inv}, std::true_type{});
+        else launch(MulDx{inv}, std::false_type{});
     } else {
-        if (wide) RENDER(DivDx, true, DivDx{s.dx});
-        else RENDER(DivDx, false, DivDx{s.dx});
+        if (wide) launch(DivDx{s.dx}, std::true_type{});
+        else launch(DivDx{s.dx}, std::false_type{});
     }
-#undef RENDER
     BLZ_HIP(hipGetLastError());
     BLZ_HIP(hipMemcpyAsync(host_rgb, fb, nf * sizeof(float), hipMemcpyDeviceToHost, s.stream));
     BLZ_HIP(hipStreamSynchronize(s.stream));
