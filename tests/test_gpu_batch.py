@@ -76,12 +76,12 @@ def test_batch_equals_single_scenes(tune):
     assert st.graph_nodes > 0
 
 
-@pytest.mark.parametrize("variant", [None, 203, 1104, 1204])
+@pytest.mark.parametrize("variant", [None, 103, 203, 1104, 1204])
 def test_batch_large_scenes_equal_single_scenes(variant):
     """Grids of 128^3 and 96x80x112 (loads from HBM, 28-32 slab groups per
     column) through the multi-grid sweep and residual kernels: every scene
     equals the same scene stepped alone bit for bit. variant None: the
-    default multi-grid sweep."""
+    default, several sweeps per launch."""
     print(f"[batch-large] variant {variant}", flush=True)
     cases = [scene(r, 20 + i) for i, r in enumerate([(128, 128, 128), (96, 80, 112)])]
     b = B.Batch([c[0] for c in cases])
@@ -104,6 +104,30 @@ def test_batch_large_scenes_equal_single_scenes(variant):
     for i in range(len(cases)):
         for w in (B.FIELD_T, B.FIELD_U, B.FIELD_V, B.FIELD_W, B.FIELD_P):
             compare(f"batch-large scene {i} field {w}", b.scenes[i].field(w), singles[i].field(w))
+
+
+@pytest.mark.parametrize("every,variant", [(2, 103), (4, 2000)])
+def test_batch_check_spacing_and_default_sweeps(every, variant):
+    """Checks two sweeps apart leave no room for several sweeps per launch: the
+    batch sweeps with the one-row fused kernel."""
+    print(f"[batch-spacing] every {every}", flush=True)
+    cases = [scene(r, 60 + i) for i, r in enumerate(SHAPES)]
+    for s, _ in cases:
+        s.residual_check_every, s.max_iter_solve, s.residual_tol = every, 40, 1e-5
+    b = B.Batch([c[0] for c in cases])
+    assert b.stats().variant == variant
+    singles = [B.Solver(c[0]) for c in cases]
+    for i, (s, part) in enumerate(cases):
+        b.scenes[i].add_source(part)
+        singles[i].add_source(part)
+    for step in range(2):
+        b.step(0.0)
+        for i, g in enumerate(singles):
+            g.step(0.0)
+            assert b.scenes[i].stats().rbgs_iters == g.stats().rbgs_iters, (step, i)
+    for i, g in enumerate(singles):
+        for w in (B.FIELD_T, B.FIELD_U, B.FIELD_V, B.FIELD_W, B.FIELD_P):
+            compare(f"batch-spacing scene {i} field {w}", b.scenes[i].field(w), g.field(w))
 
 
 def test_batch_mixed_stages_equal_single_scenes():
@@ -182,14 +206,14 @@ def test_single_grid_autotune_keeps_results():
     compare(f"autotuned v{v}", g.field(B.FIELD_P), o.field(B.FIELD_P))
 
 
-@pytest.mark.parametrize("variant", [None, 1204])
+@pytest.mark.parametrize("variant", [None, 103, 1204])
 def test_batch_with_warm_start_and_handle_steps(variant):
     """With the learned warm start inside the captured graph, each scene still
     equals the same scene stepped alone with the same network; afterwards a
     scene handle stepped on its own (outside the graph, wind noise from its
     time argument) stays equal to the single solver. variant: the batch's
-    sweep variant (None: the default one-row fused sweep; 1204: row-pair,
-    also used by each scene's warm-start judge)."""
+    sweep variant (None: the default, several sweeps per launch; 103: one-row
+    fused; 1204: row-pair; also used by each scene's warm-start judge)."""
     print(f"[batch] warm start variant {variant}", flush=True)
     net = B.Net(seed=4)
     cases = [scene(r, 10 + i) for i, r in enumerate(SHAPES[:3])]

@@ -118,7 +118,9 @@ def test_tile_sweeps_exact_division(kind, res):
 
 
 @pytest.mark.parametrize("sizes", [((32, 24, 20), (16, 40, 9)), ((96, 88, 12), (130, 66, 7)),
-                                   ((162, 133, 8), (34, 36, 16))], ids=["small", "middle", "large"])
+                                   ((162, 133, 8), (34, 36, 16)), ((200, 98, 6), (162, 133, 5)),
+                                   ((162, 133, 8), (162, 133, 5), (34, 36, 16)), ((274, 258, 5), (34, 36, 30))],
+                         ids=["small", "middle", "16x8", "16x12", "16x16", "over-256-tiles"])
 def test_batch_tile_sweeps_equal_single_scenes(sizes):
     """Scenes of unlike sizes share a tile in the batch and each get what
     they get alone; the variant can be set by its number."""
