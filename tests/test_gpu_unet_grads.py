@@ -1,5 +1,5 @@
 """GPU tests of the U-Net's weight gradients at the edges of their layout: rows
-padded to 8 elements and copied 64 at a time, the reduction over 32-element
+padded to 8 elements and copied 128 elements at a time, the reduction over 32-element
 chunks split over waves and workgroups (4 and more chunks per wave). Against
 the CPU oracle, with test_gpu_unet.py's tolerances (set before the first
 run): the operands are the same BF16 values there and the sums in float64."""
@@ -15,9 +15,10 @@ from test_gpu_unet import B, GRAD_RTOL, U, rel_l2, sample  # noqa: E402
 pytestmark = pytest.mark.gpu
 
 
-# the smallest grid (coarsest level one voxel), a row of just over 64, grids
-# with three different sides, and one whose waves take more than four chunks
-@pytest.mark.parametrize("shape", [(3, 4, 4, 4), (1, 4, 8, 68), (2, 12, 4, 20), (1, 20, 12, 8), (2, 32, 32, 32)])
+# the smallest grid (coarsest level one voxel), rows over half a copied run and
+# just over a whole one, grids with three different sides, and one whose waves
+# take more than four chunks
+@pytest.mark.parametrize("shape", [(3, 4, 4, 4), (1, 4, 8, 68), (1, 4, 8, 132), (2, 12, 4, 20), (1, 20, 12, 8), (2, 32, 32, 32)])
 def test_gradients_at_layout_edges(shape):
     print(f"[unet] gradients {shape}", flush=True)
     net = B.Net(seed=13)
