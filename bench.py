@@ -30,7 +30,7 @@ RBGS_BYTES_PER_VOXEL_SWEEP = 12.0  # read p, read rhs, write p
 RBGS_KERNELS = {1: ("k_rbgs_pass", "RBGS colour pass, two per sweep", "rbgs_pass_traffic.json"),
                 2: ("k_rbgs_fused", "RBGS fused sweep, one per sweep", "rbgs_fused_traffic.json"),
                 3: ("k_rbgs_pair", "RBGS row-pair fused sweep, one per sweep", "rbgs_pair_traffic.json"),
-                4: ("k_rbgs_tile", "RBGS tile sweeps, two to five per launch", "")}
+                4: ("k_rbgs_tile", "RBGS tile sweeps, two to five per launch", "rbgs_tile_traffic.json")}
 # compulsory bytes per voxel of the non-solve part of a substep of this
 # workload: cooling 8, vorticity 24, buoyancy 12, divergence 16, update 28,
 # advection 40 (T, U, V, W, density)
@@ -603,7 +603,7 @@ def report(a, s, gen, parts, L, LT, warm):
         "stage_ms": {B.STAGE_NAMES[i]: stage_ms[i] for i in range(B.NUM_STAGES) if stage_ms[i] > 0},
         "roofline": {
             "kernel": f"{kname} ({kdesc})",
-            "bound": "hbm",
+            "bound": "lds and hbm" if kernel_kind == 4 else "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
