@@ -72,7 +72,9 @@ __device__ __forceinline__ void advect_pair_cell(const Gv& U, const Gv& V, const
 
 // Every advected field of a grid in one launch, the longest first (a launch
 // per field left most CUs idle at 32^3: 33 us for four, 11 together; at 256^3
-// with smoke 2310 and 2100)
+// with smoke 2310 and 2100). Held to the registers of six waves per SIMD, which
+// spills 4 to 8 of a lane's (20 to 24 bytes of scratch): 2103 us against 2158
+// unbound, and 2336 at seven waves.
 struct AdvAll {
     Gv U, V, W, T, D;
     float *oT, *oD, *oF[3];

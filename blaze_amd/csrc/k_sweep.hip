@@ -15,21 +15,26 @@
 // one-sweep kernels, whatever the tile.
 //
 // What bounds it: on small grids the step (LDS reads, one dependent chain of
-// four updates, an LDS write, a barrier: about 0.45 us); on large ones LDS
-// and VALU issue in about equal parts. So half sweeps are spread over waves
+// four updates, an LDS write, a barrier: about 0.45 us). At 256^3 no one unit:
+// of a launch of two sweeps the LDS is busy for 53% (nearly half of that in
+// bank conflicts) and the vector units issue for 41%, it moves 5.6 TB/s, and a
+// wave waits half of its time. So half sweeps are spread over waves
 // (items of 64 columns) rather than walked one after the other by the wave
 // that owns a column: the first build of this kernel, a column per lane for
 // all sweeps, took 9.8 us per sweep at 128^3 (8x8 columns, 3 sweeps) against
-// 6.9 now. Measured and dropped: two slab groups per step (6.9 against 7.1
+// 6.9. Measured and dropped: two slab groups per step (6.9 against 7.1
 // us at 128^3, 20.4 against 28.9 at 256^3), old pressure and rhs 6 or 8
 // groups ahead instead of 2 or 4 (no difference), each LDS plane's pitch
 // chosen against bank conflicts (5% fewer conflicts in a model of them).
+// (These on constant pressure.)
 //
-// us per sweep (times per launch / sweeps), one sweep per launch (the
-// autotuner's pick) -> here:
-//   32^3 7.1 -> 2.6, 64^3 10.8 -> 3.6, 90x75x62 12.0 -> 4.1, 96^3 15.0 ->
-//   5.8, 128^3 20.7 -> 6.9, 192^3 29.8 -> 13.9, 256^3 41.6 -> 18 (19 where
-//   checks every 10 sweeps cut them 3 + 3 + 2 + 2).
+// us per sweep on random pressure, best kernel of one sweep per launch -> here
+// in calls of 10 (3 + 3 + 2 + 2) / of 120 sweeps:
+//   32^3 6.9 -> 3.5 / 2.7, 64^3 10.7 -> 5.0 / 3.8, 90x75x62 11.9 -> 4.9 / 4.3,
+//   96^3 14.8 -> 6.7 / 6.0, 128^3 20.6 -> 7.9 / 7.1, 192^3 29.8 -> 15.8 / 13.9,
+//   256^3 40.6 -> 23.2 / 22.9, 512^3 388 -> 231 / 253.
+// In the solves of the 256^3 explosion 22.7, the events around each call's
+// launches included.
 #include "solver.h"
 
 namespace blz {
@@ -429,8 +434,11 @@ int go(hipStream_t st, const FusedScene* one, const FusedScene* tab, int n, int 
 }
 
 // The tiles in use: columns, the most sweeps of a launch, and how many are
-// usual. From 16x8 on two: three need two items per wave, and at 256^3 a launch
-// of three takes 57 us, one of two 35.
+// usual. From 16x8 on two, as three need two items per wave: us per sweep of
+// two / three per launch on random pressure 144^3 10.0 / 11.0, 192^3 13.9 /
+// 16.8, 256^3 22.9 / 23.0; in the 256^3 explosion's solves a launch of two takes
+// 42 us and one of three 69. Three win where the planes outgrow the 256 MB
+// Infinity Cache (320^3 73 / 63, 512^3 253 / 216).
 struct Family {
     int bx, by, tmax, usual;
 };
@@ -505,12 +513,12 @@ Plan plan_of(int family, int sweeps) {
 
 // The tile for a W x H slab: the smallest of which every CU (256) gets at most
 // one; a smaller tile has more rim to compute again and takes turns, a larger
-// one leaves CUs idle. us per sweep of 4x4 / 8x4 / 8x8 / 16x16 tiles (all
-// with three sweeps per launch from 8x4 on): 64^3 3.6 / 4.0 / 4.4 / 6.8,
-// 90x75x62 4.9 / 4.1 / 4.6 / 6.9, 128^3 10.7 / 7.8 / 6.9 / 11.1. Of 8x8 /
-// 16x8 / 16x12 / 16x16 (8x8 with three, the others with two): 144^3 14.2 /
-// 10.0 / - / 13.1, 160^3 15.4 / 10.8 / - / 14.2, 192^3 25.7 / 16.8 / 13.9 /
-// 16.5, 256x128x256 22.1 / 15.4 / - / 20.7.
+// one leaves CUs idle. us per sweep on random pressure, calls of 120 sweeps, of
+// 4x4 / 8x4 / 8x8 / 16x16 tiles: 64^3 3.8 / 4.1 / 4.5 / 7.3, 90x75x62 5.3 / 4.3 /
+// 4.8 / 7.4, 128^3 15.3 / 8.0 / 7.1 / 11.8; of 8x8 / 16x8 / 16x12 / 16x16: 144^3
+// 14.2 / 10.0 / 11.2 / 13.0, 160^3 15.5 / 10.8 / 12.0 / 14.1, 192^3 26.1 / 16.9 /
+// 13.9 / 16.3, 256x128x256 22.4 / 15.5 / 17.4 / 20.4; of the last three: 224^3
+// 20.4 / 25.1 / 18.8, 256^3 25.3 / 29.4 / 22.9.
 int tile_family(int W, int H) {
     for (int f = 0; f < TILE_FAMILIES - 1; ++f)
         if (tile_count(f, W, H) <= 256) return f;
